@@ -1,37 +1,50 @@
-// Projections of many rows at once (a prompt's prefill): y = x W^T over M
-// rows as a tiled GEMM on the matrix cores, one launch per projection.
+// Projections of many rows at once (a prompt's prefill, a server's batch):
+// y = x W^T over M rows as a tiled GEMM on the matrix cores, for bf16 weights
+// and for 8-bit ones (int8 or fp8-e4m3fn codes with an fp32 scale per row).
 //
-// The multi-row kernel of gemm_rows.hip streams each weight once for up to
-// 128 rows and re-reads the rows' fragments per 16-column strip; past a few
-// hundred rows the arithmetic, not the weight stream, is the work, and a
-// 2-D tiling that reuses both operands from LDS does it with far fewer
-// instructions per multiply:
-//
-//  * block = 256 threads (2 x 2 waves) on a 128-row x 128-column output tile;
-//    each 64-deep k step stages the x tile (128 rows x 128 bytes) and the
-//    weight tile (128 rows x 128 bytes) into LDS with LDS-direct loads
-//    (16 KB each; chunk c of row r at column c ^ (r & 7), so the fragment
-//    reads of eight consecutive lanes hit eight different column groups),
-//    the next step's loads in flight during this step's multiplies, one
-//    barrier per step;
-//  * each wave multiplies a 64 x 64 quarter: D^T = W X^T on
-//    v_mfma_f32_16x16x32_bf16 (weight rows as M, x rows as N), so a lane
-//    ends with four consecutive output columns of one row (8-byte stores);
-//  * SwiGLU tiles interleave gate and up rows (32 of each per wave), so a
-//    lane holds the gate and up dot products of the same outputs;
-//  * when the 128-row grid would leave CUs without a block (short prompts),
-//    tiles take 64 x rows (each wave a 32 x 64 part), twice the blocks over
-//    the same weight tiles;
-//  * when the tiles fill at most half of the blocks the CUs hold at once
-//    (prompts of a few hundred rows; the K-long down projection most of
-//    all), each tile's k range splits over up to 8 blocks, as many as fit in
-//    one round of resident blocks; they store fp32 partial sums and a second
-//    launch adds them in split order and applies the epilogue;
+//  * block = four waves on an output tile of TM rows x 128 weight rows. The
+//    waves stand 2 x 2 (TM = 32 NT: each wave 16 NT rows x 64 weight rows) or,
+//    for at most 48 rows, 1 x 4 (TM = 16 NT: all rows x 32 weight rows);
+//  * each 64-deep k step stages the x tile (TM rows x 128 bytes) and the
+//    weight tile (128 rows of 128 bytes, or 64 for 8-bit codes) into LDS with
+//    LDS-direct loads, a ring of kStages steps deep: as many as leave room for
+//    two blocks per CU, because what bounds a few hundred rows is the weight
+//    stream, i.e. the bytes in flight, and what bounds more is the matrix
+//    cores, which need a second block's waves while one waits at its barrier.
+//    A wave waits only for the step it is about to multiply (vmcnt counts the
+//    later steps' loads, the same number in every step: steps past the end
+//    are loaded through an empty descriptor, as zeros);
+//  * x chunk c (16 bytes) of row r sits at column c ^ (r & 7), weight chunk c
+//    of an 8-bit row at c ^ ((r >> 2) & 3), so the fragment reads of eight
+//    consecutive lanes hit eight different column groups;
+//  * D^T = W X^T on v_mfma_f32_16x16x32_bf16 (weight rows as M, x rows as N):
+//    a lane ends with four consecutive output columns of one row (8-byte
+//    stores). 8-bit codes become bf16 in registers (exact for both formats)
+//    after one 16-byte read per lane and step: lane quad q holds k
+//    16 q .. 16 q + 15 and x is read in the same permuted order, which leaves
+//    each dot product unchanged. The row scale multiplies the fp32 sum, as in
+//    the batch-one GEMVs;
+//  * SwiGLU tiles interleave gate and up rows in groups of 16 (32 with 2 x 2
+//    waves), so a lane holds the gate and up dot products of the same outputs;
+//  * when the tiles leave block slots empty, each tile's k range splits over
+//    up to 8 blocks; they store fp32 partial sums and a second launch adds
+//    them in split order and applies the epilogue (with the next RMSNorm, when
+//    the caller wants it);
 //  * blocks are laid out XCD-major: the blocks of one weight tile share an
 //    XCD (block L runs on XCD L % 8), so its L2 serves the tile to all of them.
 //
 // Epilogues keep the batch-one GEMV's bf16 boundaries (store, + residual,
-// SwiGLU); fp32 accumulation over k in 64-wide steps.
+// SwiGLU, argmax keys); fp32 accumulation over k in 64-wide steps.
+//
+// Measured per 8B layer at 201 rows, bf16, against two 128-row launches of the
+// strips (gemm_rows.hip): QKV 99 -> 28 us, O 72 -> 24 (with the next norm),
+// gate/up 190 -> 67 (605 TFLOP/s, 3.0 TB/s), down 170 -> 51; 0.6B at 100 rows
+// 10 / 13 / 12 / 14 -> 8 / 10 / 8 / 11. 4B at 300 rows, fp8, against the GEMV
+// row by row: 8.4 ms -> 23 + 25 + 42 + 39 us (gate/up 712 TFLOP/s). What bounds
+// them: a CU takes 50 GB/s from HBM and 85-110 from L2 into LDS, whatever the
+// ring's depth, so a tile's staged bytes, (TM + 128) x 128 per step, set the
+// time of a step (18 KB for 16 rows: 0.36 us; 36 KB for 160: 0.9), which is
+// why few rows want narrow tiles on every CU and many want wide ones.
 #include "common.h"
 
 namespace htn {
@@ -41,209 +54,205 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_ptr_t;
 
-constexpr int kTm = 128;                  // x rows per block (64 for short prompts)
-constexpr int kTn = 128;                  // weight rows per block
 constexpr int kTk = 64;                   // k per staged step
+constexpr int kMaxTm = 256;               // x rows per block, at most
+constexpr int kCuLds = 160 * 1024;        // a CU's LDS
+constexpr int kMaxNormCols = 8192;        // a row the finish with the norm holds in LDS
 
 struct TileArgs {
   const bf16_t* x; long x_rs;
-  const bf16_t* w;
+  const unsigned char* w;
+  const float* scale;  // 8-bit weights: one per weight row
   const bf16_t* res; long res_rs;
   bf16_t* y; long y_rs;
   int M, N, K;        // N: output columns (gate columns for SwiGLU)
   int mtiles, ntiles; // output tiles along M and N
   int ksplit, steps;  // k splits per tile, 64-wide k steps per split
+  int wide;           // y rows take 8-byte stores
   float* part;        // K-split partial sums [ksplit][M][part_rs]
   long part_rs;       // round4(N), twice that for SwiGLU (gate, then up sums)
+  uint64_t* keys;     // argmax: [ntiles][M]
+  // Residual epilogue fused with the next RMSNorm (K-split finish only).
+  const bf16_t* ngain; float neps;
+  bf16_t* normed;
 };
 
-constexpr int kMinSplitSteps = 16;    // k steps each split keeps at least
-constexpr int kMaxSplit = 8;
+// k steps between the starts of neighbouring weight tiles' ranges: weight rows
+// a power of two apart (8 KB at K = 4096) put one k step's rows of every tile
+// on a few memory channels while all blocks walk k together. A copy of this
+// staging alone, 268 MB in 256 tiles: all from k = 0 4.4 TB/s, rotated 6.05,
+// rotated and past the caches (one row tile) 6.7.
+constexpr int kRotate = 37;
+constexpr int kMinSplitSteps = 8;     // k steps each split keeps at least
+constexpr int kMaxSplit = 12;
 
-// Eight 16-byte operand fragments in one asm block: LDS-direct data is read by
-// inline asm (the compiler would wait for every load in flight before an
-// ordinary LDS read of such a buffer). The reads of the next k half are issued
-// before the multiplies of this one; the wait names the fragments as
-// operands, so no use of them moves above it.
-__device__ __forceinline__ void issue_frag8(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
-                                            uint32_t a4, uint32_t a5, uint32_t a6, uint32_t a7,
-                                            u32x4 (&f)[8]) {
-  asm volatile(
-      "ds_read_b128 %0, %8\n\t"
-      "ds_read_b128 %1, %9\n\t"
-      "ds_read_b128 %2, %10\n\t"
-      "ds_read_b128 %3, %11\n\t"
-      "ds_read_b128 %4, %12\n\t"
-      "ds_read_b128 %5, %13\n\t"
-      "ds_read_b128 %6, %14\n\t"
-      "ds_read_b128 %7, %15"
-      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]),
-        "=&v"(f[6]), "=&v"(f[7])
-      : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(a4), "v"(a5), "v"(a6), "v"(a7)
-      : "memory");
+// A tile's shape: waves along the rows (2: 2 x 2 waves; 1: 1 x 4), 16-row x
+// tiles per wave, weight format.
+template <int WM, int WN, int NT, int WF>
+struct Shape {
+  static constexpr int kTm = 16 * NT * WM;
+  static constexpr int kWaves = WM * WN;
+  static constexpr int kWt = 2 * WM;                       // 16-row weight tiles per wave
+  static constexpr int kTn = 16 * kWt * WN;                // weight rows per block
+  static constexpr int kXl = (kTm / 8 + kWaves - 1) / kWaves;  // staging loads per wave: x
+  static constexpr int kWl = WF == WF_BF16 ? 4 : 2;        // and weights
+  static constexpr int kWRow = WF == WF_BF16 ? 128 : 64;   // bytes of a staged weight row
+  static constexpr int kXBytes = kTm * kTk * 2;
+  static constexpr int kStage = kXBytes + kTn * kWRow;
+  static constexpr int kBlocks = kWaves == 8 ? 1 : 2;      // resident per CU
+  static constexpr int kFit = kCuLds / kBlocks / kStage;
+  static constexpr int kStages = kFit < 2 ? 2 : (kFit > 8 ? 8 : kFit);
+};
+
+// Operand fragments are read by inline asm: the compiler would wait for every
+// LDS-direct load in flight before an ordinary LDS read of such a buffer.
+// Reads are issued without their wait; wait_frags waits and names every
+// fragment as an operand, so no use of one moves above it.
+template <int OFF>
+__device__ __forceinline__ void issue_frag(uint32_t addr, u32x4& f) {
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(f) : "v"(addr), "n"(OFF) : "memory");
 }
 
-__device__ __forceinline__ void wait_frag8(u32x4 (&f)[8]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]),
-                 "+v"(f[6]), "+v"(f[7])
-               :
-               : "memory");
+template <int N, int STRIDE, int I = 0>
+__device__ __forceinline__ void issue_frags(uint32_t addr, u32x4* f) {
+  if constexpr (I < N) {
+    issue_frag<I * STRIDE>(addr, f[I]);
+    issue_frags<N, STRIDE, I + 1>(addr, f);
+  }
 }
 
-// Six fragments (64-row tiles: four weight, two x), as issue_frag8 / wait_frag8.
-__device__ __forceinline__ void issue_frag6(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
-                                            uint32_t a4, uint32_t a5, u32x4 (&f)[6]) {
-  asm volatile(
-      "ds_read_b128 %0, %6\n\t"
-      "ds_read_b128 %1, %7\n\t"
-      "ds_read_b128 %2, %8\n\t"
-      "ds_read_b128 %3, %9\n\t"
-      "ds_read_b128 %4, %10\n\t"
-      "ds_read_b128 %5, %11"
-      : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5])
-      : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(a4), "v"(a5)
-      : "memory");
-}
-
-__device__ __forceinline__ void wait_frag6(u32x4 (&f)[6]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5])
-               :
-               : "memory");
-}
-
-// 4 x NT multiplies of one k half: weight fragments f[0..3] x x fragments
-// f[4 .. 4 + NT - 1].
-template <int NT, int NF>
-__device__ __forceinline__ void mfma_half(const u32x4 (&f)[NF], f32x4_t (&acc)[4][NT]) {
+template <int N>
+__device__ __forceinline__ void wait_frags(u32x4 (&f)[N]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[0]) : : "memory");
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          __builtin_bit_cast(bf16x8_t, f[i]), __builtin_bit_cast(bf16x8_t, f[4 + t]), acc[i][t], 0,
-          0, 0);
+  for (int i = 1; i < N; ++i) asm volatile("" : "+v"(f[i]) : : "memory");
 }
 
-__device__ __forceinline__ void lds_barrier_t() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// Epilogue of one wave's 64 x 64 quarter. Lane (col, quad) holds, per weight
-// tile i and x tile t, the outputs of x row mb + 16 t + col and weight rows
-// (output columns) nb + 16 i + 4 quad + (0..3); for SwiGLU tiles 0, 1 are the
-// gate and 2, 3 the up rows of output columns nb .. nb + 31.
-template <int EPI, int NT>
-__device__ __forceinline__ void store_tile(const TileArgs& a, const f32x4_t (&acc)[4][NT], int mb,
-                                           int nb, int col, int quad) {
-  constexpr bool SW = EPI == HTN_EPI_SWIGLU;
+// Eight 8-bit codes (k ascending) as eight bf16 values, exactly.
+template <int WF>
+__device__ __forceinline__ u32x4 codes_to_bf16(uint32_t lo, uint32_t hi) {
+  u32x4 o;
+  const uint32_t d[2] = {lo, hi};
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int m = mb + 16 * t + col;
-    if (m >= a.M) continue;
-    if constexpr (SW) {
-      // Weight tiles 0, 1 are gate columns nb .. nb + 31 and 2, 3 the up
-      // columns of the same outputs.
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int n = nb + 16 * i + 4 * quad;
-        if (n >= a.N) continue;
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          o[e] = silu_bf(round_bf(acc[i][t][e])) * round_bf(acc[i + 2][t][e]);
-        bf16_t* dst = a.y + static_cast<long>(m) * a.y_rs + n;
-        if (n + 4 <= a.N) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
-        } else {
-          for (int e = 0; e < 4 && n + e < a.N; ++e) dst[e] = static_cast<bf16_t>(f2bf(o[e]));
-        }
-      }
+  for (int j = 0; j < 2; ++j) {
+    if constexpr (WF == WF_INT8) {
+      const int v = static_cast<int>(d[j]);
+      o[2 * j] = pack_exact_bf2(static_cast<float>(static_cast<signed char>(v)),
+                                static_cast<float>(static_cast<signed char>(v >> 8)));
+      o[2 * j + 1] = pack_exact_bf2(static_cast<float>(static_cast<signed char>(v >> 16)),
+                                    static_cast<float>(v >> 24));
     } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = nb + 16 * i + 4 * quad;
-        if (n >= a.N) continue;
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          o[e] = acc[i][t][e];
-          if (EPI == HTN_EPI_RESIDUAL)
-            o[e] = round_bf(o[e]) + (n + e < a.N ? bf2f(a.res[static_cast<long>(m) * a.res_rs + n + e]) : 0.f);
-        }
-        bf16_t* dst = a.y + static_cast<long>(m) * a.y_rs + n;
-        if (n + 4 <= a.N) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
-        } else {
-          for (int e = 0; e < 4 && n + e < a.N; ++e) dst[e] = static_cast<bf16_t>(f2bf(o[e]));
-        }
-      }
+      o[2 * j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                                                  static_cast<int>(d[j]), 1.0f, false));
+      o[2 * j + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                                                      static_cast<int>(d[j]), 1.0f, true));
     }
+  }
+  return o;
+}
+
+__device__ __forceinline__ f32x4_t mfma(u32x4 w, u32x4 x, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w),
+                                                 __builtin_bit_cast(bf16x8_t, x), c, 0, 0, 0);
+}
+
+// The fp32 dot products of output columns n .. n + 3 (weight rows row0 + n ..):
+// 8-bit weights' row scales applied.
+template <int WF>
+__device__ __forceinline__ f32x4_t scaled(const TileArgs& a, f32x4_t v, int row0, int n) {
+  if constexpr (WF != WF_BF16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] *= n + e < a.N ? a.scale[row0 + n + e] : 0.f;
+  }
+  return v;
+}
+
+// Four output columns n .. n + 3 of row m (fewer at the right edge).
+__device__ __forceinline__ void store4(const TileArgs& a, int m, int n, const float (&o)[4]) {
+  bf16_t* dst = a.y + static_cast<long>(m) * a.y_rs + n;
+  if (a.wide && n + 4 <= a.N) {
+    *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < a.N) dst[e] = static_cast<bf16_t>(f2bf(o[e]));
   }
 }
 
-// K-split epilogue: the block's fp32 sums of its k range, unrounded, at
-// part[(s M + m) part_rs + c], c = the output column, or for SwiGLU c = n for
-// the gate sums and part_rs / 2 + n for the up sums of output column n. The
-// four columns of a lane end before round4(N), so every store is whole.
-template <bool SW, int NT>
-__device__ __forceinline__ void store_part(const TileArgs& a, const f32x4_t (&acc)[4][NT], int s,
-                                           int mb, int nb, int col, int quad) {
+// The epilogue of four outputs: g holds the (gate) dot products, u the up ones.
+template <int EPI, int WF>
+__device__ __forceinline__ void finish4(const TileArgs& a, int m, int n, f32x4_t g, f32x4_t u) {
+  g = scaled<WF>(a, g, 0, n);
+  float o[4];
+  if constexpr (EPI == HTN_EPI_SWIGLU) {
+    u = scaled<WF>(a, u, a.N, n);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int m = mb + 16 * t + col;
-    if (m >= a.M) continue;
-    float* row = a.part + (static_cast<long>(s) * a.M + m) * a.part_rs;
+    for (int e = 0; e < 4; ++e) o[e] = silu_bf(round_bf(g[e])) * round_bf(u[e]);
+  } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = nb + 16 * (SW ? (i & 1) : i) + 4 * quad;
-      if (n >= a.N) continue;
-      *reinterpret_cast<f32x4_t*>(row + (SW && i >= 2 ? a.part_rs / 2 : 0) + n) = acc[i][t];
+    for (int e = 0; e < 4; ++e) {
+      o[e] = g[e];
+      if (EPI == HTN_EPI_RESIDUAL)
+        o[e] = round_bf(o[e]) +
+               (n + e < a.N ? bf2f(a.res[static_cast<long>(m) * a.res_rs + n + e]) : 0.f);
     }
+  }
+  store4(a, m, n, o);
+}
+
+// A uniform pointer kept in scalar registers: a descriptor in vector registers
+// makes every load through it a per-lane descriptor loop.
+__device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char* ptr) {
+  const uint64_t p = reinterpret_cast<uint64_t>(ptr);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
+  return reinterpret_cast<const unsigned char*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// One k step into ring slot `slot` (empty past the split's last step): eight x
+// rows (1 KB) per load, weight rows eight (bf16) or sixteen (8-bit) per load.
+template <int WM, int WN, int NT, int WF, int AUX>
+__device__ __forceinline__ void stage_tiles(unsigned char* st, int ks, bool live, int wave,
+                                            const bf16_t* xb, uint32_t xrange,
+                                            const unsigned char* const (&wb)[2],
+                                            const uint32_t (&wrange)[2],
+                                            const uint32_t* xoff,
+                                            const uint32_t (&woff)[2]) {
+  using S = Shape<WM, WN, NT, WF>;
+  const uint32_t kx = live ? static_cast<uint32_t>(ks) * kTk * 2u : 0u;
+  const uint32_t kw = live ? static_cast<uint32_t>(ks) * S::kWRow : 0u;
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xb, live ? xrange : 0u);
+#pragma unroll
+  for (int u = 0; u < S::kXl; ++u) {
+    int li = wave + S::kWaves * u;  // where loads and waves do not divide, some repeat
+    if ((S::kTm / 8) % S::kWaves != 0) li %= S::kTm / 8;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr_t*)(st + li * 1024), 16, xoff[u], kx, 0, 0);
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {  // the wave's two 16-row groups of the weight tile
+    const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(wb[h], live ? wrange[h] : 0u);
+    unsigned char* dst = st + S::kXBytes + (2 * wave + h) * 16 * S::kWRow;
+#pragma unroll
+    for (int u = 0; u < S::kWl / 2; ++u)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_ptr_t*)(dst + u * 1024), 16, woff[u], kw, 0, AUX);
   }
 }
 
-// Bytes of one staged k step: the x tile (TM rows) and the weight tile (128
-// rows), 128 bytes per row.
-template <int TM>
-struct Stage {
-  static constexpr int kBytes = (TM + kTn) * kTk * 2;
-};
-
-// One k step into its stage: wave w's x rows (TM / 4 of them) and weight rows
-// (32), eight rows (1 KB) per LDS-direct load.
-template <int TM>
-__device__ __forceinline__ void stage_tiles(unsigned char* lds, int ks, int wave,
-                                            __amdgpu_buffer_rsrc_t xrs, __amdgpu_buffer_rsrc_t wrs,
-                                            const uint32_t (&xoff)[4],
-                                            const uint32_t (&woff)[4]) {
-  unsigned char* st = lds + (ks & 1) * Stage<TM>::kBytes;
-  const uint32_t ko = static_cast<uint32_t>(ks) * kTk * 2u;
-#pragma unroll
-  for (int u = 0; u < TM / 32; ++u)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_ptr_t*)(st + ((TM / 4) * wave + 8 * u) * 128),
-                                             16, xoff[u], ko, 0, 0);
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        wrs, (lds_ptr_t*)(st + TM * kTk * 2 + (32 * wave + 8 * u) * 128), 16, woff[u], ko, 0, 0);
-}
-
-template <int EPI, int TM>
-__global__ __launch_bounds__(256) void gemm_tiles_kernel(TileArgs a) {
+template <int EPI, int WM, int WN, int NT, int WF>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tiles_kernel(TileArgs a) {
+  using S = Shape<WM, WN, NT, WF>;
+  constexpr bool SW = EPI == HTN_EPI_SWIGLU;
+  constexpr int WT = S::kWt, TM = S::kTm;
+  // Weights of a single row tile are read once: streamed past the caches.
+  constexpr int AUX = WM == 1 ? 2 : 0;
   // Arguments in scalar registers at entry: one round of scalar loads.
-  asm volatile("" ::"s"(a.x), "s"(a.x_rs), "s"(a.w), "s"(a.res), "s"(a.res_rs), "s"(a.y),
-               "s"(a.y_rs), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.mtiles), "s"(a.ntiles),
+  asm volatile("" ::"s"(a.x), "s"(a.x_rs), "s"(a.w), "s"(a.scale), "s"(a.res), "s"(a.res_rs),
+               "s"(a.y), "s"(a.y_rs), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.mtiles), "s"(a.ntiles),
                "s"(a.ksplit), "s"(a.steps), "s"(a.part), "s"(a.part_rs));
-  extern __shared__ __align__(16) unsigned char lds[];  // two stages of x and weight tiles
-  constexpr int NT = TM / 32;        // 16-row x tiles per wave (4 or 2)
-  constexpr int XR = TM / 4;         // x rows each wave stages (32 or 16)
-  constexpr int kStage = Stage<TM>::kBytes;
-  constexpr int kXBytes = TM * kTk * 2;
+  extern __shared__ __align__(16) unsigned char lds[];  // kStages x and weight tiles
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;  // this wave's TM / 2 x rows, 64 weight rows
+  const int wm = WM == 2 ? wave & 1 : 0, wn = WM == 2 ? wave >> 1 : wave;
   const int col = lane & 15, quad = lane >> 4;
   // XCD-major layout: block L on XCD L % 8 takes weight tile
   // nt = (L / 8 / (mtiles ksplit)) * 8 + L % 8, row tile (L / 8) % mtiles and
@@ -254,119 +263,217 @@ __global__ __launch_bounds__(256) void gemm_tiles_kernel(TileArgs a) {
   if (nt >= a.ntiles) return;
   const int m0 = mt * TM;
   // Weight rows of the tile: rows n0 .. n0 + 127, or for SwiGLU 64 output
-  // columns c0 .. c0 + 63 as four 32-row groups gate, up, gate, up.
-  constexpr bool SW = EPI == HTN_EPI_SWIGLU;
-  const int n0 = SW ? nt * 64 : nt * kTn;
+  // columns n0 .. n0 + 63 as eight 16-row groups: gate, gate, up, up, twice
+  // (2 x 2 waves), or gate, up, four times.
+  const int n0 = nt * (SW ? S::kTn / 2 : S::kTn);
 
-  // Staging: wave w loads x rows XR w .. XR w + XR - 1 and weight rows 32 w ..
-  // 32 w + 31 of the tile, eight rows (1 KB) per instruction; lane l takes
-  // row 8 u + l / 8 of the wave's rows and writes position l % 8 of it,
-  // loading source chunk (l % 8) ^ (row & 7). Both operands go through one
-  // descriptor per wave whose range ends at the last real row, so rows past
-  // M or past the weight's end read as zeros. For SwiGLU, wave w's 32 weight
-  // rows are group w: gate, up, gate, up rows of columns n0 + 32 (w / 2) ...
-  const int lr = lane >> 3, lp = lane & 7;
+  // Staging: a lane of load li takes x row 8 li + lane / 8 and writes position
+  // lane % 8 of it, loading source chunk (lane % 8) ^ (row & 7); weights the
+  // same, or for 8-bit rows 16 rows per load, row lane / 4, chunk
+  // (lane % 4) ^ ((row >> 2) & 3). Operands go through descriptors whose range
+  // ends at the last real row, so rows past M or the weight's end read zeros.
   const long mrows = a.M - m0 < TM ? a.M - m0 : TM;
-  const __amdgpu_buffer_rsrc_t xrs =
-      buffer_rsrc(a.x + static_cast<long>(m0) * a.x_rs,
-                  static_cast<uint32_t>(mrows * a.x_rs * 2));
-  long wbase, wrows;
-  if (SW) {
-    const int c0 = n0 + (wave >> 1) * 32;
-    wbase = static_cast<long>((wave & 1) ? a.N : 0) + c0;
-    wrows = a.N - c0 < 32 ? (a.N - c0 > 0 ? a.N - c0 : 0) : 32;
-  } else {
-    wbase = n0 + 32 * wave;
-    wrows = a.N - wbase < 32 ? (a.N - wbase > 0 ? a.N - wbase : 0) : 32;
-  }
-  const __amdgpu_buffer_rsrc_t wrs = uniform_rsrc(a.w + (wrows > 0 ? wbase : 0) * a.K,
-                                                  static_cast<uint32_t>(wrows * a.K * 2));
-  uint32_t xoff[4], woff[4];  // x offsets: the first TM / 32 are used
-#pragma unroll
-  for (int u = 0; u < XR / 8; ++u) {
-    const int r = XR * wave + 8 * u + lr;  // x tile row
-    xoff[u] = static_cast<uint32_t>(r) * static_cast<uint32_t>(a.x_rs) * 2u + (lp ^ (r & 7)) * 16;
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int c = 8 * u + lr;     // row within the wave's 32
-    const int r = 32 * wave + c;  // weight tile row
-    woff[u] = static_cast<uint32_t>(c) * static_cast<uint32_t>(a.K) * 2u + (lp ^ (r & 7)) * 16;
-  }
-
-  // Fragment addresses in stage 0 (stage 1 is kStage further): k chunk
-  // 4 h + quad of row 16 t + col, un-swizzled.
-  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t*)lds));
-  uint32_t wa[2][4], xa[2][NT];  // [k half][tile]
+  const bf16_t* xb = a.x + static_cast<long>(m0) * a.x_rs;
+  const uint32_t xrange = static_cast<uint32_t>(((mrows - 1) * a.x_rs + a.K) * 2);
+  const long wrow_bytes = static_cast<long>(a.K) * (WF == WF_BF16 ? 2 : 1);
+  const unsigned char* wb[2];
+  uint32_t wrange[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int rw = 64 * wn + 16 * t + col;
-      wa[h][t] = base + kXBytes + static_cast<uint32_t>(rw * 128 + ((((4 * h + quad) ^ (rw & 7))) * 16));
+    const int gi = 2 * wave + h;
+    int first = n0 + 16 * gi, base = first;  // output column, weight row
+    if (SW) {
+      first = WM == 2 ? n0 + 32 * (gi >> 2) + 16 * (gi & 1) : n0 + 16 * (gi >> 1);
+      base = first + ((WM == 2 ? (gi & 2) : (gi & 1)) ? a.N : 0);
     }
+    const int rows = a.N - first < 16 ? (a.N - first > 0 ? a.N - first : 0) : 16;
+    wb[h] = uniform_ptr(a.w + (rows > 0 ? base : 0) * wrow_bytes);
+    wrange[h] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(rows * wrow_bytes));
+  }
+  uint32_t xoff[S::kXl], woff[2];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int rx = (TM / 2) * wm + 16 * t + col;
-      xa[h][t] = base + static_cast<uint32_t>(rx * 128 + ((((4 * h + quad) ^ (rx & 7))) * 16));
-    }
+  for (int u = 0; u < S::kXl; ++u) {
+    int li = wave + S::kWaves * u;
+    if ((TM / 8) % S::kWaves != 0) li %= TM / 8;
+    const int r = 8 * li + (lane >> 3);
+    xoff[u] = static_cast<uint32_t>(r) * static_cast<uint32_t>(a.x_rs) * 2u +
+              (((lane & 7) ^ (r & 7)) * 16);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = WF == WF_BF16 ? 8 * u + (lane >> 3) : (lane >> 2);
+    woff[u] = static_cast<uint32_t>(r) * static_cast<uint32_t>(wrow_bytes) +
+              (WF == WF_BF16 ? ((lane & 7) ^ (r & 7)) * 16 : ((lane & 3) ^ ((r >> 2) & 3)) * 16);
   }
 
-  f32x4_t acc[4][NT];  // [weight tile][x tile]: D^T rows = weight rows, columns = x rows
+  // Fragment addresses in ring slot 0, per k half: x and bf16 weights, chunk
+  // 4 h + quad (8-bit: 2 quad + h) of row 16 t + col; 8-bit weights, chunk
+  // quad, both halves in one read. Row tiles are 2048 (1024) bytes apart.
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t*)lds));
+  uint32_t xa[2], wa[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int h = 0; h < 2; ++h) {
+    const int c = WF == WF_BF16 ? 4 * h + quad : 2 * quad + h;
+    xa[h] = lds0 + static_cast<uint32_t>((16 * NT * wm + col) * 128 + ((c ^ (col & 7)) * 16));
+    wa[h] = lds0 + S::kXBytes +
+            static_cast<uint32_t>(WF == WF_BF16
+                                      ? (16 * WT * wn + col) * 128 + ((c ^ (col & 7)) * 16)
+                                      : (16 * WT * wn + col) * 64 + ((quad ^ ((col >> 2) & 3)) * 16));
+  }
+
+  f32x4_t acc[WT][NT];  // [weight tile][x tile]: D^T rows = weight rows, columns = x rows
+#pragma unroll
+  for (int i = 0; i < WT; ++i)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int nk = a.K / kTk;
   const int k0 = s * a.steps, k1 = nk < k0 + a.steps ? nk : k0 + a.steps;
-  stage_tiles<TM>(lds, k0, wave, xrs, wrs, xoff, woff);
+  int left = k1 - k0;                  // steps still to stage
+  int kn = k0 + (nt * kRotate) % left;  // the next one
+  auto stage_next = [&](int slot) {
+    stage_tiles<WM, WN, NT, WF, AUX>(lds + slot * S::kStage, kn, left > 0, wave, xb, xrange, wb,
+                                       wrange, xoff, woff);
+    kn = kn + 1 == k1 ? k0 : kn + 1;
+    --left;
+  };
+#pragma unroll
+  for (int u = 0; u < S::kStages - 1; ++u) stage_next(u);
+  int rd = 0, wr = S::kStages - 1;
   for (int ks = k0; ks < k1; ++ks) {
-    // This wave's part of step ks has landed; after the barrier everyone's
-    // has, and every wave has finished step ks - 1, whose stage step ks + 1
-    // now takes (in flight during this step's multiplies).
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier_t();
-    if (ks + 1 < k1) stage_tiles<TM>(lds, ks + 1, wave, xrs, wrs, xoff, woff);
-    const uint32_t so = static_cast<uint32_t>((ks & 1) * kStage);
-    if constexpr (NT == 4) {
-      u32x4 f0[8], f1[8];
-      issue_frag8(wa[0][0] + so, wa[0][1] + so, wa[0][2] + so, wa[0][3] + so, xa[0][0] + so,
-                  xa[0][1] + so, xa[0][2] + so, xa[0][3] + so, f0);
-      wait_frag8(f0);
-      issue_frag8(wa[1][0] + so, wa[1][1] + so, wa[1][2] + so, wa[1][3] + so, xa[1][0] + so,
-                  xa[1][1] + so, xa[1][2] + so, xa[1][3] + so, f1);
+    // This wave's part of step ks has landed (the later steps' loads may still
+    // be in flight); after the barrier everyone's has, and every wave has
+    // finished step ks - 1, whose slot the next load takes.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S::kStages - 2) * (S::kXl + S::kWl)) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+    stage_next(wr);
+    const uint32_t so = static_cast<uint32_t>(rd * S::kStage);
+    rd = rd + 1 == S::kStages ? 0 : rd + 1;
+    wr = wr + 1 == S::kStages ? 0 : wr + 1;
+    if constexpr (WF == WF_BF16) {
+      u32x4 f0[WT + NT], f1[WT + NT];
+      issue_frags<WT, 2048>(wa[0] + so, f0);
+      issue_frags<NT, 2048>(xa[0] + so, f0 + WT);
+      wait_frags(f0);
+      issue_frags<WT, 2048>(wa[1] + so, f1);
+      issue_frags<NT, 2048>(xa[1] + so, f1 + WT);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_half<NT>(f0, acc);
+#pragma unroll
+      for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = mfma(f0[i], f0[WT + t], acc[i][t]);
       __builtin_amdgcn_sched_barrier(0);
-      wait_frag8(f1);
-      mfma_half<NT>(f1, acc);
+      wait_frags(f1);
+#pragma unroll
+      for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = mfma(f1[i], f1[WT + t], acc[i][t]);
     } else {
-      u32x4 f0[6], f1[6];
-      issue_frag6(wa[0][0] + so, wa[0][1] + so, wa[0][2] + so, wa[0][3] + so, xa[0][0] + so,
-                  xa[0][1] + so, f0);
-      wait_frag6(f0);
-      issue_frag6(wa[1][0] + so, wa[1][1] + so, wa[1][2] + so, wa[1][3] + so, xa[1][0] + so,
-                  xa[1][1] + so, f1);
+      u32x4 f0[WT + NT], f1[NT];  // codes of both halves and x of the first; x of the second
+      issue_frags<WT, 1024>(wa[0] + so, f0);
+      issue_frags<NT, 2048>(xa[0] + so, f0 + WT);
+      wait_frags(f0);
+      issue_frags<NT, 2048>(xa[1] + so, f1);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_half<NT>(f0, acc);
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const u32x4 w = codes_to_bf16<WF>(f0[i][0], f0[i][1]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = mfma(w, f0[WT + t], acc[i][t]);
+      }
       __builtin_amdgcn_sched_barrier(0);
-      wait_frag6(f1);
-      mfma_half<NT>(f1, acc);
+      wait_frags(f1);
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const u32x4 w = codes_to_bf16<WF>(f0[i][2], f0[i][3]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = mfma(w, f1[t], acc[i][t]);
+      }
     }
   }
+  // Every staging load has landed before the block's LDS is reused or released.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  const int mb = m0 + (TM / 2) * wm, nb = SW ? n0 + 32 * wn : n0 + 64 * wn;
-  if (a.ksplit > 1)
-    store_part<SW, NT>(a, acc, s, mb, nb, col, quad);
-  else
-    store_tile<EPI, NT>(a, acc, mb, nb, col, quad);
+  // Lane (col, quad) holds, per weight tile i and x tile t, row mb + 16 t + col
+  // and weight rows 16 (WT wn + i) + 4 quad + (0..3) of the tile; for SwiGLU
+  // the first half of a wave's weight tiles are gate, the second up rows.
+  const int mb = m0 + 16 * NT * wm;
+  constexpr int OT = SW ? WT / 2 : WT;  // 16-column output tiles per wave
+  const int nb = n0 + 16 * OT * wn + 4 * quad;
+  if constexpr (EPI == HTN_EPI_ARGMAX) {
+    // The best (bf16 logit, lowest id) key of the tile's columns per row: over
+    // the lane's columns, the four quads, then the waves.
+    uint64_t* best = reinterpret_cast<uint64_t*>(lds);  // [4 waves][NT * 16]
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      uint64_t key = 0;
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const f32x4_t v = scaled<WF>(a, acc[i][t], 0, nb + 16 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int n = nb + 16 * i + e;
+          const uint64_t k = n < a.N ? argmax_key(f2bf(v[e]), static_cast<uint32_t>(n)) : 0ull;
+          key = k > key ? k : key;
+        }
+      }
+#pragma unroll
+      for (int d = 16; d <= 32; d += d) {
+        const uint64_t o = __shfl_xor(key, d, kWave);
+        key = o > key ? o : key;
+      }
+      if (quad == 0) best[wave * (NT * 16) + 16 * t + col] = key;
+    }
+    __syncthreads();
+    for (int r = tid; r < TM; r += 64 * S::kWaves) {
+      const int w0 = WM == 2 ? r / (16 * NT) : 0, rr = r - w0 * 16 * NT;
+      uint64_t key = 0;
+      for (int w = w0; w < 4; w += WM) {
+        const uint64_t k = best[w * (NT * 16) + rr];
+        key = k > key ? k : key;
+      }
+      if (m0 + r < a.M) a.keys[static_cast<long>(nt) * a.M + m0 + r] = key;
+    }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int m = mb + 16 * t + col;
+    if (m >= a.M) continue;
+    // K-split partials, unrounded and unscaled, at part[(s M + m) part_rs + c],
+    // c = the output column, or for SwiGLU c = n for the gate sums and
+    // part_rs / 2 + n for the up sums. The four columns of a lane end before
+    // round4(N), so every store is whole.
+    float* row = a.part + (static_cast<long>(s) * a.M + m) * a.part_rs;
+#pragma unroll
+    for (int i = 0; i < OT; ++i) {
+      const int n = nb + 16 * i;
+      if (n >= a.N) continue;
+      const f32x4_t u = SW ? acc[SW ? i + OT : i][t] : f32x4_t{};
+      if (a.ksplit > 1) {
+        *reinterpret_cast<f32x4_t*>(row + n) = acc[i][t];
+        if (SW) *reinterpret_cast<f32x4_t*>(row + a.part_rs / 2 + n) = u;
+      } else {
+        finish4<EPI, WF>(a, m, n, acc[i][t], u);
+      }
+    }
+  }
 }
 
-// K-split sum + epilogue: thread i takes output columns 4 (i % (part_rs' / 4))
-// .. + 3 of row i / (part_rs' / 4) (part_rs' = round4(N)), adds the splits'
-// partials in split order and rounds as store_tile does.
-template <int EPI>
+// The k splits' partial sums of columns n .. n + 3 of row m, in split order.
+__device__ __forceinline__ f32x4_t sum_parts(const TileArgs& a, long m, long n) {
+  const long stride = static_cast<long>(a.M) * a.part_rs;
+  const float* p = a.part + m * a.part_rs + n;
+  f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
+#pragma unroll 4
+  for (int s = 1; s < a.ksplit; ++s) v += *reinterpret_cast<const f32x4_t*>(p + s * stride);
+  return v;
+}
+
+// K-split sum + epilogue: thread i takes output columns 4 (i % n4) .. + 3 of
+// row i / n4, n4 = round4(N) / 4.
+template <int EPI, int WF>
 __global__ __launch_bounds__(256) void gemm_tiles_finish(TileArgs a) {
   asm volatile("" ::"s"(a.res), "s"(a.res_rs), "s"(a.y), "s"(a.y_rs), "s"(a.M), "s"(a.N),
                "s"(a.ksplit), "s"(a.part), "s"(a.part_rs));
@@ -376,94 +483,285 @@ __global__ __launch_bounds__(256) void gemm_tiles_finish(TileArgs a) {
   const long m = i / n4;
   if (m >= a.M) return;
   const int n = static_cast<int>(i - m * n4) * 4;
-  const long stride = static_cast<long>(a.M) * a.part_rs;
-  const float* p = a.part + m * a.part_rs + n;
-  f32x4_t g = *reinterpret_cast<const f32x4_t*>(p), u{};
-  if (SW) u = *reinterpret_cast<const f32x4_t*>(p + a.part_rs / 2);
-  for (int s = 1; s < a.ksplit; ++s) {
-    g += *reinterpret_cast<const f32x4_t*>(p + s * stride);
-    if (SW) u += *reinterpret_cast<const f32x4_t*>(p + s * stride + a.part_rs / 2);
+  const f32x4_t g = sum_parts(a, m, n);
+  const f32x4_t u = SW ? sum_parts(a, m, a.part_rs / 2 + n) : f32x4_t{};
+  finish4<EPI, WF>(a, static_cast<int>(m), n, g, u);
+}
+
+// K-split finish of the residual epilogue with the next RMSNorm, one block per
+// row: y = bf16(bf16(sum) + residual) to memory and LDS, then wave 0 forms the
+// sum of squares in the row-wise RMSNorm's order (lane l over vectors l,
+// l + 64, ..., element by element, one wave reduction), so `normed` is
+// bit-identical to running that norm on y.
+template <int WF>
+__global__ __launch_bounds__(256) void gemm_tiles_finish_norm(TileArgs a) {
+  asm volatile("" ::"s"(a.res), "s"(a.res_rs), "s"(a.y), "s"(a.y_rs), "s"(a.M), "s"(a.N),
+               "s"(a.ksplit), "s"(a.part), "s"(a.part_rs), "s"(a.ngain), "s"(a.neps),
+               "s"(a.normed));
+  __shared__ uint4 ys[kMaxNormCols / 8];
+  __shared__ float inv_s;
+  const int tid = threadIdx.x, m = blockIdx.x, nv = a.N >> 3;
+  for (int v = tid; v < nv; v += 256) {
+    const f32x4_t t0 = scaled<WF>(a, sum_parts(a, m, 8 * v), 0, 8 * v);
+    const f32x4_t t1 = scaled<WF>(a, sum_parts(a, m, 8 * v + 4), 0, 8 * v + 4);
+    float r[8];
+    unpack8(*reinterpret_cast<const uint4*>(a.res + m * a.res_rs + v * 8), r);
+    uint4 yv;
+    yv.x = pack_bf2(round_bf(t0[0]) + r[0], round_bf(t0[1]) + r[1]);
+    yv.y = pack_bf2(round_bf(t0[2]) + r[2], round_bf(t0[3]) + r[3]);
+    yv.z = pack_bf2(round_bf(t1[0]) + r[4], round_bf(t1[1]) + r[5]);
+    yv.w = pack_bf2(round_bf(t1[2]) + r[6], round_bf(t1[3]) + r[7]);
+    *reinterpret_cast<uint4*>(a.y + m * a.y_rs + v * 8) = yv;
+    ys[v] = yv;
   }
-  float o[4];
+  __syncthreads();
+  if (tid < kWave) {
+    float ss = 0.f;
+    for (int v = tid; v < nv; v += kWave) {
+      float f[8];
+      unpack8(ys[v], f);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (SW)
-      o[e] = silu_bf(round_bf(g[e])) * round_bf(u[e]);
-    else if (EPI == HTN_EPI_RESIDUAL)
-      o[e] = round_bf(g[e]) + (n + e < a.N ? bf2f(a.res[m * a.res_rs + n + e]) : 0.f);
-    else
-      o[e] = g[e];
+      for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
+    }
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(a.N) + a.neps);
+    if (tid == 0) inv_s = inv;
   }
-  bf16_t* dst = a.y + m * a.y_rs + n;
-  if (n + 4 <= a.N) {
-    *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
-  } else {
-    for (int e = 0; e < 4 && n + e < a.N; ++e) dst[e] = static_cast<bf16_t>(f2bf(o[e]));
+  __syncthreads();
+  const float inv = inv_s;
+  for (int v = tid; v < nv; v += 256)
+    *reinterpret_cast<uint4*>(a.normed + static_cast<long>(m) * a.N + v * 8) =
+        norm8(ys[v], *reinterpret_cast<const uint4*>(a.ngain + v * 8), inv);
+}
+
+// Per-row argmax over the weight tiles' keys.
+__global__ __launch_bounds__(256) void gemm_tiles_argmax(const uint64_t* __restrict__ keys,
+                                                         int tiles, int M, int64_t* tokens) {
+  __shared__ uint64_t wbest[4];
+  const int m = blockIdx.x;
+  uint64_t b = 0;
+  for (int i = threadIdx.x; i < tiles; i += 256) {
+    const uint64_t k = keys[static_cast<long>(i) * M + m];
+    b = k > b ? k : b;
+  }
+  b = wave_max_u64(b);
+  if ((threadIdx.x & 63) == 0) wbest[threadIdx.x >> 6] = b;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t r = wbest[0];
+    for (int i = 1; i < 4; ++i) r = wbest[i] > r ? wbest[i] : r;
+    tokens[m] = static_cast<int64_t>(argmax_key_index(r));
   }
 }
 
-// Launch shape: the row tile (128, or 64 when the 128-row grid would leave
-// CUs without a block: twice the blocks over the same weight tiles; 8B
-// 256-token prefill 14.9 -> 13.9 ms, at a full first wave of 128-row blocks
-// the 64-row tiles measured slower) and the k split.
+// Launch shape: the row tile, and the k split.
 struct TilePlan {
-  int tm, ksplit, steps;
-  long blocks, part_rs;
+  int wm, wn, nt;     // waves along the rows and the weight rows, 16-row tiles per wave
+  int ksplit, steps;
+  long blocks, ntiles, part_rs, keys_bytes;
 };
 
-TilePlan plan_tiles(long rows, long n, long k, int epilogue) {
-  const bool sw = epilogue == HTN_EPI_SWIGLU;
-  const long cols = (((sw ? (n + 63) / 64 : (n + kTn - 1) / kTn) + 7) / 8) * 8;
-  const long cus = device_cus();
-  TilePlan p{};
-  p.tm = cols * ((rows + 127) / 128) < cus ? 64 : 128;
-  const long base = cols * ((rows + p.tm - 1) / p.tm);
+// The tiles and what one k step of a block on them takes, in us, alone on its
+// CU (step[0]) and beside a second block (step[1]; eight waves stand alone):
+// bf16, then 8-bit weights. Measured over the QKV, O, gate/up and down
+// projections of the 0.6B, 4B and 8B shapes at 5 to 1000 rows, every tile with
+// 1 to 12 k splits (1200 launches, weights from HBM), as the coefficients that
+// fit those times best; the plan below then picks launches 1% slower than the
+// fastest of each sweep on average, 16% at most.
+struct TileShape { int wm, wn, nt; float step[2][2]; };
+constexpr TileShape kShapes[] = {
+    {1, 4, 1, {{.36f, .72f}, {.32f, .68f}}}, {1, 4, 2, {{.38f, .84f}, {.35f, .78f}}},
+    {1, 4, 3, {{.45f, .94f}, {.41f, .89f}}}, {2, 2, 2, {{.47f, .81f}, {.47f, .73f}}},
+    {2, 2, 3, {{.80f, .93f}, {.59f, .83f}}}, {2, 2, 4, {{.85f, 1.08f}, {.69f, .97f}}},
+    {2, 2, 5, {{.89f, 1.16f}, {.84f, 1.08f}}}, {2, 4, 4, {{.96f, .96f}, {1.06f, 1.06f}}},
+    {2, 4, 5, {{1.11f, 1.11f}, {1.20f, 1.20f}}}, {2, 4, 7, {{1.50f, 1.50f}, {1.52f, 1.52f}}},
+    {2, 4, 8, {{1.54f, 1.54f}, {1.68f, 1.68f}}}};
+
+// A launch's time by those coefficients: per XCD, `blocks` blocks of `steps`
+// k steps in rounds of two per CU (one, for eight waves), the launch itself,
+// and for a k split its finish: a launch, the partial sums' bytes, and for
+// the finish with a norm (a block per row) its chain over the splits.
+float tile_cost(const TileShape& sh, long blocks, long steps, long ks, double part_mb,
+                bool residual, int format) {
+  const long cus = device_cus() / 8 > 0 ? device_cus() / 8 : 1;
+  const long per = cus * (sh.wm * sh.wn == 8 ? 1 : 2);
+  const float* step = sh.step[format != 0];
+  const long rest = blocks % per;
+  float t = blocks / per * step[1];
+  if (rest > 0) t += rest <= cus ? step[0] : step[1];
+  t = t * steps + 3.3f;
+  if (ks > 1) t += 2.6f + .43f * static_cast<float>(part_mb) + (residual ? .64f * ks : 0.f);
+  else if (residual) t += 6.4f;  // the norm's own launch
+  return t;
+}
+
+TilePlan plan_tiles(long rows, long n, long k, int epilogue, int format) {
+  const bool sw = epilogue == HTN_EPI_SWIGLU, argmax = epilogue == HTN_EPI_ARGMAX;
   const long nk = k / kTk;
-  // Blocks resident at once: 64-row tiles take 48 KB of the CU's 160 KB of
-  // LDS (three blocks), 128-row tiles 64 KB (two). A split that overflows
-  // one round of them measured slower (8B QKV at 1024 rows: 384 -> 768
-  // blocks of 128 rows, 74 -> 87 us).
-  const long slots = cus * (p.tm == 64 ? 3 : 2);
-  long ks = 1;
-  if (2 * base <= slots) {
-    ks = slots / base;
-    if (ks > nk / kMinSplitSteps) ks = nk / kMinSplitSteps;
-    if (ks > kMaxSplit) ks = kMaxSplit;
-    if (ks < 1) ks = 1;
-  }
-  p.steps = static_cast<int>((nk + ks - 1) / ks);
-  p.ksplit = static_cast<int>((nk + p.steps - 1) / p.steps);
-  p.blocks = base * p.ksplit;
+  // bf16 prompts whose 128 x 128 tiles alone give every CU its two blocks keep
+  // whole k ranges: their callers need no scratch.
+  const bool full = format == 0 && ((rows + 127) / 128) * ((n * (sw ? 2 : 1) + 127) / 128) >=
+                                       2L * device_cus();
+  TilePlan p{};
   p.part_rs = (sw ? 2 : 1) * ((n + 3) / 4 * 4);
+  float best = 0.f;
+  for (const TileShape& sh : kShapes) {
+    if (argmax && (sh.wm != 1 || sh.nt > 2)) continue;
+    const long tm = 16L * sh.nt * sh.wm, tn = 32L * sh.wm * sh.wn / (sw ? 2 : 1);
+    const long ntiles = (n + tn - 1) / tn;
+    const long per_xcd = (ntiles + 7) / 8 * ((rows + tm - 1) / tm);
+    for (long ks = 1; ks <= kMaxSplit; ++ks) {
+      if (ks > 1 && (argmax || full || nk / ks < kMinSplitSteps)) break;
+      const long steps = (nk + ks - 1) / ks;
+      if ((nk + steps - 1) / steps != ks) continue;  // a split would be empty
+      const float cost = tile_cost(sh, per_xcd * ks, steps, ks, ks * rows * p.part_rs * 4e-6,
+                                   epilogue == HTN_EPI_RESIDUAL, format);
+      if (p.ksplit == 0 || cost < best) {
+        best = cost;
+        p.wm = sh.wm; p.wn = sh.wn; p.nt = sh.nt;
+        p.ntiles = ntiles;
+        p.ksplit = static_cast<int>(ks);
+        p.steps = static_cast<int>(steps);
+        p.blocks = 8 * per_xcd * ks;
+      }
+    }
+  }
+  p.keys_bytes = argmax ? p.ntiles * rows * 8 : 0;
   return p;
 }
 
 long tiles_scratch_bytes(const TilePlan& p, long rows) {
-  return p.ksplit > 1 ? static_cast<long>(p.ksplit) * rows * p.part_rs * 4 : 0;
+  return p.ksplit > 1 ? static_cast<long>(p.ksplit) * rows * p.part_rs * 4 : p.keys_bytes;
 }
 
-template <int EPI, int TM>
-int launch_tiles(TileArgs& a, long blocks, hipStream_t st) {
-  const size_t lds = 2 * static_cast<size_t>(Stage<TM>::kBytes);
+template <int EPI, int WM, int WN, int NT, int WF>
+int launch_shape(TileArgs& a, long blocks, hipStream_t st) {
+  using S = Shape<WM, WN, NT, WF>;
+  constexpr int bytes = S::kStages * S::kStage;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&gemm_tiles_kernel<EPI, TM>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+      reinterpret_cast<const void*>(&gemm_tiles_kernel<EPI, WM, WN, NT, WF>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   (void)attr;  // a refused size surfaces as a launch error
-  a.mtiles = static_cast<int>((a.M + TM - 1) / TM);
-  hipLaunchKernelGGL((gemm_tiles_kernel<EPI, TM>), dim3(static_cast<unsigned>(blocks)), dim3(256),
-                     lds, st, a);
+  a.mtiles = (a.M + S::kTm - 1) / S::kTm;
+  hipLaunchKernelGGL((gemm_tiles_kernel<EPI, WM, WN, NT, WF>), dim3(static_cast<unsigned>(blocks)),
+                     dim3(64 * S::kWaves), bytes, st, a);
   return launch_status();
 }
 
-template <int EPI>
-int launch_tiles_for(TileArgs& a, const TilePlan& p, hipStream_t st) {
-  const int rc = p.tm == 64 ? launch_tiles<EPI, 64>(a, p.blocks, st)
-                            : launch_tiles<EPI, 128>(a, p.blocks, st);
-  if (rc != HTN_OK || a.ksplit == 1) return rc;
+template <int EPI, int WF>
+int launch_tiles(TileArgs& a, const TilePlan& p, hipStream_t st) {
+  if constexpr (EPI == HTN_EPI_ARGMAX) {
+    return p.nt == 1 ? launch_shape<EPI, 1, 4, 1, WF>(a, p.blocks, st)
+                     : launch_shape<EPI, 1, 4, 2, WF>(a, p.blocks, st);
+  } else {
+    switch (100 * p.wm + 10 * p.wn + p.nt) {
+      case 141: return launch_shape<EPI, 1, 4, 1, WF>(a, p.blocks, st);
+      case 142: return launch_shape<EPI, 1, 4, 2, WF>(a, p.blocks, st);
+      case 143: return launch_shape<EPI, 1, 4, 3, WF>(a, p.blocks, st);
+      case 222: return launch_shape<EPI, 2, 2, 2, WF>(a, p.blocks, st);
+      case 223: return launch_shape<EPI, 2, 2, 3, WF>(a, p.blocks, st);
+      case 224: return launch_shape<EPI, 2, 2, 4, WF>(a, p.blocks, st);
+      case 225: return launch_shape<EPI, 2, 2, 5, WF>(a, p.blocks, st);
+      case 244: return launch_shape<EPI, 2, 4, 4, WF>(a, p.blocks, st);
+      case 245: return launch_shape<EPI, 2, 4, 5, WF>(a, p.blocks, st);
+      case 247: return launch_shape<EPI, 2, 4, 7, WF>(a, p.blocks, st);
+      default: return launch_shape<EPI, 2, 4, 8, WF>(a, p.blocks, st);
+    }
+  }
+}
+
+template <int EPI, int WF>
+int finish_tiles(TileArgs& a, hipStream_t st) {
   const long groups = static_cast<long>(a.M) * ((a.N + 3) / 4);
-  hipLaunchKernelGGL((gemm_tiles_finish<EPI>), dim3(static_cast<unsigned>((groups + 255) / 256)),
+  hipLaunchKernelGGL((gemm_tiles_finish<EPI, WF>), dim3(static_cast<unsigned>((groups + 255) / 256)),
                      dim3(256), 0, st, a);
   return launch_status();
+}
+
+template <int WF>
+int run_tiles(TileArgs& a, const TilePlan& p, int epilogue, int64_t* tokens, hipStream_t st) {
+  int rc;
+  switch (epilogue) {
+    case HTN_EPI_STORE: rc = launch_tiles<HTN_EPI_STORE, WF>(a, p, st); break;
+    case HTN_EPI_RESIDUAL: rc = launch_tiles<HTN_EPI_RESIDUAL, WF>(a, p, st); break;
+    case HTN_EPI_SWIGLU: rc = launch_tiles<HTN_EPI_SWIGLU, WF>(a, p, st); break;
+    default: rc = launch_tiles<HTN_EPI_ARGMAX, WF>(a, p, st); break;
+  }
+  if (rc != HTN_OK) return rc;
+  if (epilogue == HTN_EPI_ARGMAX) {
+    hipLaunchKernelGGL(gemm_tiles_argmax, dim3(a.M), dim3(256), 0, st, a.keys, a.ntiles, a.M, tokens);
+    return launch_status();
+  }
+  if (a.ksplit == 1) return HTN_OK;
+  if (a.normed) {
+    hipLaunchKernelGGL((gemm_tiles_finish_norm<WF>), dim3(a.M), dim3(256), 0, st, a);
+    return launch_status();
+  }
+  switch (epilogue) {
+    case HTN_EPI_STORE: return finish_tiles<HTN_EPI_STORE, WF>(a, st);
+    case HTN_EPI_RESIDUAL: return finish_tiles<HTN_EPI_RESIDUAL, WF>(a, st);
+    default: return finish_tiles<HTN_EPI_SWIGLU, WF>(a, st);
+  }
+}
+
+bool known_epilogue(int e, int format) {
+  return e == HTN_EPI_STORE || e == HTN_EPI_RESIDUAL || e == HTN_EPI_SWIGLU ||
+         (e == HTN_EPI_ARGMAX && format != 0);
+}
+
+int tiles(const void* x, int64_t x_stride, const void* w, const float* scale, int format, int64_t n,
+          int64_t k, int64_t rows, int epilogue, const void* residual, int64_t res_stride, void* y,
+          int64_t y_stride, const void* gain, float eps, void* normed, int64_t* tokens,
+          void* scratch, hipStream_t st) {
+  if (!x || !w || rows <= 0 || n <= 0 || k <= 0) return HTN_EINVAL;
+  if (format < 0 || format > HTN_WEIGHT_FP8_E4M3 || (format != 0 && !scale)) return HTN_EINVAL;
+  if (!known_epilogue(epilogue, format)) return HTN_EINVAL;
+  const bool argmax = epilogue == HTN_EPI_ARGMAX;
+  if (argmax ? !tokens : !y) return HTN_EINVAL;
+  if (epilogue == HTN_EPI_RESIDUAL && (!residual || res_stride < n)) return HTN_EINVAL;
+  if ((!argmax && y_stride < n) || x_stride < k) return HTN_EINVAL;  // rows must not overlap
+  // 64-wide k steps of 16-byte chunks; 32-bit offsets.
+  if (k % kTk || k > (1L << 20) || x_stride % 8 || !aligned16(x) || !aligned16(w))
+    return HTN_EUNSUPPORTED;
+  const long wrows = epilogue == HTN_EPI_SWIGLU ? 2 * n : n;
+  if (static_cast<long>(kMaxTm) * x_stride * 2 >= (1L << 32) || wrows >= (1L << 31) ||
+      rows >= (1L << 31) || (argmax && rows > HTN_GEMM_TILES_ARGMAX_ROWS))
+    return HTN_EUNSUPPORTED;
+  if (!aligned16(scratch)) return HTN_EUNSUPPORTED;
+  TilePlan p = plan_tiles(rows, n, k, epilogue, format);
+  if (!scratch) {  // no scratch: every tile sums its whole k range
+    if (argmax) return HTN_EINVAL;
+    p.blocks /= p.ksplit;
+    p.ksplit = 1;
+    p.steps = static_cast<int>(k / kTk);
+  }
+  TileArgs a{};
+  a.x = static_cast<const bf16_t*>(x); a.x_rs = x_stride;
+  a.w = static_cast<const unsigned char*>(w);
+  a.scale = scale;
+  a.res = static_cast<const bf16_t*>(residual); a.res_rs = res_stride;
+  a.y = static_cast<bf16_t*>(y); a.y_rs = y_stride;
+  a.M = static_cast<int>(rows); a.N = static_cast<int>(n); a.K = static_cast<int>(k);
+  a.ntiles = static_cast<int>(p.ntiles);
+  a.ksplit = p.ksplit;
+  a.steps = p.steps;
+  a.wide = y_stride % 4 == 0 && aligned8(y);
+  a.part = static_cast<float*>(scratch);
+  a.part_rs = p.part_rs;
+  a.keys = static_cast<uint64_t*>(scratch);
+  // The finish with the norm holds a row of y in LDS as 8-element vectors.
+  const bool fused = gain && p.ksplit > 1 && n % 8 == 0 && n <= kMaxNormCols &&
+                     res_stride % 8 == 0 && y_stride % 8 == 0 && aligned16(residual) &&
+                     aligned16(y) && aligned16(gain) && aligned16(normed);
+  if (fused) {
+    a.ngain = static_cast<const bf16_t*>(gain);
+    a.neps = eps;
+    a.normed = static_cast<bf16_t*>(normed);
+  }
+  const int rc = format == 0              ? run_tiles<WF_BF16>(a, p, epilogue, tokens, st)
+                 : format == HTN_WEIGHT_INT8 ? run_tiles<WF_INT8>(a, p, epilogue, tokens, st)
+                                             : run_tiles<WF_FP8>(a, p, epilogue, tokens, st);
+  if (rc != HTN_OK || !gain || fused) return rc;
+  return htn_rms_norm(y, y_stride, gain, normed, rows, n, eps, st);
 }
 
 }  // namespace
@@ -473,51 +771,46 @@ using namespace htn;
 
 extern "C" int64_t htn_gemm_tiles_scratch_bytes(int64_t rows, int64_t n, int64_t k,
                                                 int epilogue) {
-  if (rows <= 0 || n <= 0 || k <= 0 || k % kTk) return 0;
-  if (epilogue != HTN_EPI_STORE && epilogue != HTN_EPI_RESIDUAL && epilogue != HTN_EPI_SWIGLU)
+  return htn_gemm_tiles_w8_scratch_bytes(rows, n, k, epilogue, 0);
+}
+
+extern "C" int64_t htn_gemm_tiles_w8_scratch_bytes(int64_t rows, int64_t n, int64_t k, int epilogue,
+                                                   int format) {
+  if (rows <= 0 || n <= 0 || k <= 0 || k % kTk || format < 0 || format > HTN_WEIGHT_FP8_E4M3 ||
+      !known_epilogue(epilogue, format))
     return 0;
-  return tiles_scratch_bytes(plan_tiles(rows, n, k, epilogue), rows);
+  return tiles_scratch_bytes(plan_tiles(rows, n, k, epilogue, format), rows);
 }
 
 extern "C" int htn_gemm_tiles(const void* x, int64_t x_stride, const void* w, int64_t n,
                               int64_t k, int64_t rows, int epilogue, const void* residual,
                               int64_t res_stride, void* y, int64_t y_stride, void* scratch,
                               htn_stream_t stream) {
-  if (!x || !w || !y || rows <= 0 || n <= 0 || k <= 0) return HTN_EINVAL;
-  if (epilogue != HTN_EPI_STORE && epilogue != HTN_EPI_RESIDUAL && epilogue != HTN_EPI_SWIGLU)
-    return HTN_EINVAL;
-  if (epilogue == HTN_EPI_RESIDUAL && (!residual || res_stride < n)) return HTN_EINVAL;
-  if (y_stride < n || x_stride < k) return HTN_EINVAL;  // rows must not overlap
-  // 64-wide k steps of 16-byte chunks; 8-byte output stores; 32-bit offsets.
-  if (k % kTk || k > (1L << 20) || x_stride % 8 || y_stride % 4 || !aligned16(x) || !aligned16(w) ||
-      (reinterpret_cast<uintptr_t>(y) & 7u))
-    return HTN_EUNSUPPORTED;
-  const long wrows = epilogue == HTN_EPI_SWIGLU ? 2 * n : n;
-  if (static_cast<long>(kTm) * x_stride * 2 >= (1L << 31) || k * 2 >= (1L << 31) ||
-      wrows >= (1L << 31) || rows >= (1L << 31))
-    return HTN_EUNSUPPORTED;
-  TileArgs a{};
-  a.x = static_cast<const bf16_t*>(x); a.x_rs = x_stride;
-  a.w = static_cast<const bf16_t*>(w);
-  a.res = static_cast<const bf16_t*>(residual); a.res_rs = res_stride;
-  a.y = static_cast<bf16_t*>(y); a.y_rs = y_stride;
-  a.M = static_cast<int>(rows); a.N = static_cast<int>(n); a.K = static_cast<int>(k);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  a.ntiles = static_cast<int>(epilogue == HTN_EPI_SWIGLU ? (n + 63) / 64 : (n + kTn - 1) / kTn);
-  if (!aligned16(scratch)) return HTN_EUNSUPPORTED;
-  TilePlan p = plan_tiles(rows, n, k, epilogue);
-  if (!scratch) {  // no scratch: every tile sums its whole k range
-    p.blocks /= p.ksplit;
-    p.ksplit = 1;
-    p.steps = static_cast<int>(k / kTk);
-  }
-  a.ksplit = p.ksplit;
-  a.steps = p.steps;
-  a.part = static_cast<float*>(scratch);
-  a.part_rs = p.part_rs;
-  switch (epilogue) {
-    case HTN_EPI_STORE: return launch_tiles_for<HTN_EPI_STORE>(a, p, st);
-    case HTN_EPI_RESIDUAL: return launch_tiles_for<HTN_EPI_RESIDUAL>(a, p, st);
-    default: return launch_tiles_for<HTN_EPI_SWIGLU>(a, p, st);
-  }
+  if (epilogue == HTN_EPI_ARGMAX) return HTN_EINVAL;
+  if (y_stride % 4 || !aligned8(y)) return y && y_stride >= n ? HTN_EUNSUPPORTED : HTN_EINVAL;
+  return tiles(x, x_stride, w, nullptr, 0, n, k, rows, epilogue, residual, res_stride, y, y_stride,
+               nullptr, 0.f, nullptr, nullptr, scratch, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int htn_gemm_tiles_w8(const void* x, int64_t x_stride, const void* w,
+                                 const float* w_scale, int weight_format, int64_t n, int64_t k,
+                                 int64_t rows, int epilogue, const void* residual,
+                                 int64_t res_stride, void* y, int64_t y_stride, int64_t* tokens,
+                                 void* scratch, htn_stream_t stream) {
+  if (weight_format != HTN_WEIGHT_INT8 && weight_format != HTN_WEIGHT_FP8_E4M3) return HTN_EINVAL;
+  return tiles(x, x_stride, w, w_scale, weight_format, n, k, rows, epilogue, residual, res_stride,
+               y, y_stride, nullptr, 0.f, nullptr, tokens, scratch,
+               static_cast<hipStream_t>(stream));
+}
+
+extern "C" int htn_gemm_tiles_residual_norm(const void* x, int64_t x_stride, const void* w,
+                                            const float* w_scale, int weight_format, int64_t n,
+                                            int64_t k, int64_t rows, const void* residual,
+                                            int64_t res_stride, void* y, int64_t y_stride,
+                                            const void* gain, float eps, void* normed,
+                                            void* scratch, htn_stream_t stream) {
+  if (!gain || !normed) return HTN_EINVAL;
+  return tiles(x, x_stride, w, w_scale, weight_format, n, k, rows, HTN_EPI_RESIDUAL, residual,
+               res_stride, y, y_stride, gain, eps, normed, nullptr, scratch,
+               static_cast<hipStream_t>(stream));
 }

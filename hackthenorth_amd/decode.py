@@ -25,8 +25,8 @@ from .kernels.embed import embed_gather, embed_gather_pair
 from .kernels.fused import norm_rope_cache
 from .kernels.greedy import greedy_head
 from .kernels.projection import norm_projection, output_projection_residual
-from .kernels.rows import (TILE_ROWS, greedy_rows, projection_rows, residual_norm_rows,
-                           residual_rows, splits_k, swiglu_rows)
+from .kernels.rows import (greedy_rows, projection_rows, residual_norm_rows, residual_rows,
+                           splits_k, swiglu_rows, tiled)
 from .speculate import draft_width, verified_tokens
 
 
@@ -167,8 +167,9 @@ def _attention_chunks(q, keys, values, positions, groups):
 def _forward_rows(model, token_ids, cache, positions, last_only, position_embeddings, rotary,
                   record=None):
     """Any batch and token count (prefill, verify): multi-row MFMA projections
-    that read each weight once per 32 rows, batched norm/RoPE/cache append and
-    grouped attention. 8-bit weights take the batch-one GEMVs row by row.
+    that read each weight once, batched norm/RoPE/cache append and grouped
+    attention. A single row of 8-bit weights, and widths off the tiles' 64-wide
+    steps, take the batch-one GEMVs row by row.
     `record`, when a list, receives every layer's output rows [B, T, H]."""
     c = model.config
     b, t = token_ids.shape
@@ -180,7 +181,7 @@ def _forward_rows(model, token_ids, cache, positions, last_only, position_embedd
     widths = c.widths
     groups = c.num_attention_heads // c.num_key_value_heads
     rows = b * t
-    multi = not c.quantized
+    multi = not c.quantized or (rows > 1 and hidden % 64 == 0 and c.intermediate_size % 64 == 0)
     hn = None  # the down projection's output normalised for the next layer (multi-row path)
     for i, layer in enumerate(model.layers):
         ln1, ln2 = layer.input_layernorm, layer.post_attention_layernorm
@@ -207,11 +208,10 @@ def _forward_rows(model, token_ids, cache, positions, last_only, position_embedd
                                       positions)
             a = _attention_chunks(q, cache.keys[i], cache.values[i], positions, groups)
         if multi:
-            # A projection that splits K writes the next RMSNorm in its split
-            # finish, and a prompt's projections (TILE_ROWS rows or more) write
-            # it with their residual add; otherwise the next projection
-            # normalises its rows itself.
-            if rows >= TILE_ROWS or splits_k(*layer.o_weight.shape, rows):
+            # The tiles write the next RMSNorm with their residual projections
+            # (in the split finish, where k splits), and so do strips that split
+            # K; otherwise the next projection normalises its rows itself.
+            if tiled(a, layer.o_weight) or splits_k(*layer.o_weight.shape, rows):
                 r, rn = residual_norm_rows(a, layer.o_weight, h, ln2.weight,
                                            ln2.variance_epsilon)
                 m = swiglu_rows(rn, layer.gate_up_weight)
@@ -220,7 +220,7 @@ def _forward_rows(model, token_ids, cache, positions, last_only, position_embedd
                 m = swiglu_rows(r, layer.gate_up_weight, ln2.weight, ln2.variance_epsilon)
             nxt = model.layers[i + 1].input_layernorm if i + 1 < len(model.layers) \
                 else model.norm
-            if rows >= TILE_ROWS or splits_k(*layer.down_weight.shape, rows):
+            if tiled(m, layer.down_weight) or splits_k(*layer.down_weight.shape, rows):
                 h, hn = residual_norm_rows(m, layer.down_weight, r, nxt.weight,
                                            nxt.variance_epsilon)
             else:
@@ -344,8 +344,8 @@ class DecodeState:
     def prefill(self, model, input_ids):
         """The whole prompt in one causal multi-row pass (decode.py:157-166).
 
-        Every prompt token's K/V goes to its cache slot, the projections read
-        each weight once per 32 rows, attention is causal by absolute position,
+        Every prompt token's K/V goes to its cache slot, the projections run
+        over all rows at once, attention is causal by absolute position,
         and only the last row of each sequence reaches the LM head. Afterwards
         `token` holds the greedy continuation and `position` equals the prompt
         length. Launches only: it can be captured (prefill.prefill does).

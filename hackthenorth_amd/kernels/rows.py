@@ -1,23 +1,39 @@
-"""Projections of 2 to 128 rows that read each weight once (MFMA tiles).
+"""Projections of two or more rows that read each weight once (MFMA tiles).
 
 The speculative verify pass scores k + 1 tokens in one forward; the reference
 runs its multi-row projections as Triton GEMM tiles (dryft/engine/
 projections.py:168-183, kernels/gateup.py:40-58, kernels/split_down.py:85-101).
-Here every multi-row projection is one htn_gemm_rows launch (plus a K-split
-reduction when the strips alone cannot fill the GPU) with the batch-one
-GEMVs' bf16 rounding boundaries. From TILE_ROWS rows on (a prompt's
-prefill) the plain product runs through hipBLASLt (htn_gemm_library) with
-the epilogues as row-wise launches (RMSNorm before, SwiGLU or the residual add
-with the next RMSNorm after), or, where the library has no algorithm and for
-residual projections without a following norm, as one tiled GEMM launch with
-the epilogue fused (htn_gemm_tiles); otherwise rows run in chunks of 128.
+Here up to STRIP_ROWS rows are one htn_gemm_rows launch (16-column strips, the
+RMSNorm inside, plus a K-split reduction when the strips alone cannot fill the
+GPU) and more rows one htn_gemm_tiles launch (LDS-staged output tiles, plus the
+finish of its k split), with the batch-one GEMVs' bf16 rounding boundaries.
+From TILE_ROWS rows on (a prompt's prefill) the plain product of the gate/up
+projection, and from LIBRARY_ROWS on of every projection, runs through
+hipBLASLt (htn_gemm_library) with the epilogues as row-wise launches, where the
+library has an algorithm. 8-bit weights (QuantizedWeight) take
+htn_gemm_tiles_w8 at every row count.
 """
 import torch
 
 from .. import _lib
+from ..quant import QuantizedWeight
+from .greedy import greedy_head
 
-MAX_ROWS = 128
+MAX_ROWS = 128    # rows per htn_gemm_rows launch
+# Rows up to which bf16 projections take the strips: at 16 rows of the 8B
+# shape strips / tiles take 15.6 / 13.9 us for QKV and 18 / 15 for O without
+# their norms, which the strips compute inside (a launch, 4 us), and at 5 rows
+# of the 4B the strips win outright (8.9 / 10.4, 12.2 / 13.2); at 32 rows of
+# the 8B QKV, O, gate/up and down take 21 / 15, 21 / 15, 44 / 35 and 40 / 30.
+STRIP_ROWS = 16
+ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
+# Rows from which a plain store (QKV) and a residual projection leave the
+# tiles, whose finish writes the next norm too, for the library: 8B at 300
+# rows QKV 32 us on the tiles and 30 through the library, O with its norm 29
+# and 35, down 59 and 78; at 512 rows 44 / 38, 35 / 39, 79 / 90; at 2048 the
+# library wins throughout (QKV 85 us against 137).
+LIBRARY_ROWS = 512
 # Plain products of TILE_ROWS rows or more through hipBLASLt (False: this
 # library's tiled kernel for every prompt projection, e.g. to measure it).
 LIBRARY = True
@@ -55,15 +71,12 @@ def _library(x, weight, width):
 
 def _prefill(x, weight, n, epilogue, gain=None, eps=1e-6):
     """Store or SwiGLU epilogue over every row of a prompt: the plain product
-    through the library, SwiGLU as a row-wise launch; the tiled kernel when
-    the library declines the shape."""
+    through the library, SwiGLU as a row-wise launch; the tiled kernel below
+    LIBRARY_ROWS rows of a store and when the library declines the shape."""
     xn = _normed(x, gain, eps)
     width = 2 * n if epilogue == _lib.EPI_SWIGLU else n
-    # A plain store of under 512 rows keeps the tiles' k split: the 8B QKV
-    # projection at 256 rows takes 35.5 us there against 42.4 us through the
-    # library (which wins from 512 rows on and for every other projection).
-    y = _library(xn, weight, width) if epilogue != _lib.EPI_STORE or x.shape[0] >= 2 * TILE_ROWS \
-        else None
+    y = _library(xn, weight, width) \
+        if epilogue != _lib.EPI_STORE or x.shape[0] >= LIBRARY_ROWS else None
     if y is None:
         return _tiles(xn, weight, n, epilogue)
     if epilogue == _lib.EPI_STORE:
@@ -75,19 +88,69 @@ def _prefill(x, weight, n, epilogue, gain=None, eps=1e-6):
     return out
 
 
+def _weight(weight):
+    """(bytes, row scales or None, format code) of a bf16 or 8-bit weight."""
+    if isinstance(weight, QuantizedWeight):
+        return weight.data, weight.scale, weight.code
+    return weight, None, 0
+
+
+def prompt(x, weight):
+    """Whether the library may take part: bf16 projections of TILE_ROWS rows or more."""
+    return x.shape[0] >= TILE_ROWS and not isinstance(weight, QuantizedWeight)
+
+
+def _tiles_scratch(device, rows, n, k, epilogue, fmt):
+    nbytes = _lib.load().htn_gemm_tiles_w8_scratch_bytes(rows, n, k, epilogue, fmt)
+    return torch.empty((nbytes + 15) // 16, 4, dtype=torch.float32, device=device) \
+        if nbytes > 0 else None
+
+
 def _tiles(x, weight, n, epilogue, residual=None, gain=None, eps=1e-6):
-    """One htn_gemm_tiles launch over every row of x (after the rows' RMSNorm
-    with `gain`, when given); returns the [M, n] output."""
+    """One tiled launch over every row of x (after the rows' RMSNorm with
+    `gain`, when given); returns the [M, n] output."""
     rows, k = x.shape
     x = _normed(x, gain, eps)
+    data, scale, fmt = _weight(weight)
     out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
-    nbytes = _lib.load().htn_gemm_tiles_scratch_bytes(rows, n, k, epilogue)
-    scratch = torch.empty((nbytes + 15) // 16, 4, dtype=torch.float32, device=x.device) \
-        if nbytes > 0 else None
-    _lib.call("htn_gemm_tiles", _lib.ptr(x), x.stride(0), _lib.ptr(weight), n, k, rows, epilogue,
-              _lib.ptr(residual), residual.stride(0) if residual is not None else 0,
-              _lib.ptr(out), out.stride(0), _lib.ptr(scratch), _lib.stream(x.device))
+    scratch = _tiles_scratch(x.device, rows, n, k, epilogue, fmt)
+    tail = (n, k, rows, epilogue, _lib.ptr(residual),
+            residual.stride(0) if residual is not None else 0, _lib.ptr(out), out.stride(0))
+    if fmt:
+        _lib.call("htn_gemm_tiles_w8", _lib.ptr(x), x.stride(0), _lib.ptr(data), _lib.ptr(scale),
+                  fmt, *tail, None, _lib.ptr(scratch), _lib.stream(x.device))
+    else:
+        _lib.call("htn_gemm_tiles", _lib.ptr(x), x.stride(0), _lib.ptr(data), *tail,
+                  _lib.ptr(scratch), _lib.stream(x.device))
     return out
+
+
+def _tiles_residual_norm(x, weight, residual, gain, eps):
+    """(out, normed) of a residual projection and the next RMSNorm: one launch
+    and, when the tiles split k, its finish, which writes both."""
+    rows, k = x.shape
+    n = weight.shape[0]
+    data, scale, fmt = _weight(weight)
+    out = torch.empty((rows, n), dtype=x.dtype, device=x.device)
+    normed = torch.empty_like(out)
+    scratch = _tiles_scratch(x.device, rows, n, k, _lib.EPI_RESIDUAL, fmt)
+    _lib.call("htn_gemm_tiles_residual_norm", _lib.ptr(x), x.stride(0), _lib.ptr(data),
+              _lib.ptr(scale), fmt, n, k, rows, _lib.ptr(residual), residual.stride(0),
+              _lib.ptr(out), out.stride(0), _lib.ptr(gain), float(eps), _lib.ptr(normed),
+              _lib.ptr(scratch), _lib.stream(x.device))
+    return out, normed
+
+
+def tiled(x, weight):
+    """Whether a projection of these rows takes the tiles: 8-bit weights
+    always, bf16 ones past STRIP_ROWS rows whose output rows the tiles' 8-byte
+    stores and whose input strides their 32-bit offsets cover (TILE_ROWS rows
+    or more have no other kernel)."""
+    if isinstance(weight, QuantizedWeight):
+        return True
+    rows = x.shape[0]
+    return rows >= TILE_ROWS or (rows > STRIP_ROWS and weight.shape[0] % 8 == 0
+                                 and x.stride(0) < 1 << 22)
 
 
 def _scratch(device, rows, n, k, epilogue, norm):
@@ -100,6 +163,10 @@ def _scratch(device, rows, n, k, epilogue, norm):
 def _check(x, weight):
     if x.dim() != 2 or x.dtype != torch.bfloat16 or x.stride(1) != 1:
         raise ValueError("rows must be a bf16 [M, K] matrix with unit column stride")
+    if isinstance(weight, QuantizedWeight):
+        if weight.shape[1] != x.shape[1]:
+            raise ValueError("weight must be an 8-bit [N, K] matrix matching x")
+        return
     if weight.dim() != 2 or weight.dtype != torch.bfloat16 or not weight.is_contiguous() \
             or weight.shape[1] != x.shape[1]:
         raise ValueError("weight must be a contiguous bf16 [N, K] matrix matching x")
@@ -122,9 +189,10 @@ def _chunks(rows):
 def projection_rows(x, weight, gain=None, eps=1e-6):
     """bf16(W x_m) for every row m of x [M, K]; gain applies RMSNorm first."""
     _check(x, weight)
-    _lib.require_gpu(x, weight, gain)
-    if x.shape[0] >= TILE_ROWS:
-        return _prefill(x, weight, weight.shape[0], _lib.EPI_STORE, gain=gain, eps=eps)
+    _lib.require_gpu(x, _weight(weight)[0], gain)
+    if tiled(x, weight):
+        run = _prefill if prompt(x, weight) else _tiles
+        return run(x, weight, weight.shape[0], _lib.EPI_STORE, gain=gain, eps=eps)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device)
     for s, e in _chunks(x.shape[0]):
         _launch(x[s:e], weight, weight.shape[0], _lib.EPI_STORE, gain, eps, out=out[s:e])
@@ -137,8 +205,8 @@ def residual_rows(x, weight, residual):
     if residual.shape != (x.shape[0], weight.shape[0]) or residual.dtype != torch.bfloat16 \
             or residual.stride(1) != 1:
         raise ValueError("residual must be bf16 [M, N] with unit column stride")
-    _lib.require_gpu(x, weight, residual)
-    if x.shape[0] >= TILE_ROWS:
+    _lib.require_gpu(x, _weight(weight)[0], residual)
+    if tiled(x, weight):
         return _tiles(x, weight, weight.shape[0], _lib.EPI_RESIDUAL, residual=residual)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device)
     for s, e in _chunks(x.shape[0]):
@@ -167,7 +235,9 @@ def residual_norm_rows(x, weight, residual, gain, eps=1e-6):
     if gain is None or gain.shape != (n,) or gain.dtype != torch.bfloat16 \
             or not gain.is_contiguous():
         raise ValueError("gain must be a contiguous bf16 [N] vector")
-    _lib.require_gpu(x, weight, residual, gain)
+    _lib.require_gpu(x, _weight(weight)[0], residual, gain)
+    if tiled(x, weight) and not (prompt(x, weight) and x.shape[0] > LIBRARY_ROWS):
+        return _tiles_residual_norm(x, weight, residual, gain, eps)
     if x.shape[0] >= TILE_ROWS:
         rows = x.shape[0]
         y = _library(x, weight, n)
@@ -202,10 +272,11 @@ def swiglu_rows(x, gate_up_weight, gain=None, eps=1e-6):
     _check(x, gate_up_weight)
     if gate_up_weight.shape[0] % 2:
         raise ValueError("packed gate/up width must be even")
-    _lib.require_gpu(x, gate_up_weight, gain)
+    _lib.require_gpu(x, _weight(gate_up_weight)[0], gain)
     n = gate_up_weight.shape[0] // 2
-    if x.shape[0] >= TILE_ROWS:
-        return _prefill(x, gate_up_weight, n, _lib.EPI_SWIGLU, gain=gain, eps=eps)
+    if tiled(x, gate_up_weight):
+        run = _prefill if prompt(x, gate_up_weight) else _tiles
+        return run(x, gate_up_weight, n, _lib.EPI_SWIGLU, gain=gain, eps=eps)
     out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
     for s, e in _chunks(x.shape[0]):
         _launch(x[s:e], gate_up_weight, n, _lib.EPI_SWIGLU, gain, eps, out=out[s:e])
@@ -215,8 +286,23 @@ def swiglu_rows(x, gate_up_weight, gain=None, eps=1e-6):
 def greedy_rows(x, weight, gain=None, eps=1e-6):
     """argmax_n bf16(W x_m) per row (lowest id on ties); gain applies RMSNorm first."""
     _check(x, weight)
-    _lib.require_gpu(x, weight, gain)
+    _lib.require_gpu(x, _weight(weight)[0], gain)
     tokens = torch.empty((x.shape[0],), dtype=torch.int64, device=x.device)
+    if x.shape[0] == 1 and x.is_contiguous():
+        # The batch-one head normalises in its launch and streams the weight
+        # with nothing else to do (8B: 182 us against 220).
+        return greedy_head(x, gain, eps, weight, tokens)
+    if isinstance(weight, QuantizedWeight):
+        xn = _normed(x, gain, eps)
+        n, k = weight.shape
+        for s in range(0, x.shape[0], ARGMAX_ROWS):
+            part = xn[s:s + ARGMAX_ROWS]
+            rows = part.shape[0]
+            scratch = _tiles_scratch(x.device, rows, n, k, _lib.EPI_ARGMAX, weight.code)
+            _lib.call("htn_gemm_tiles_w8", _lib.ptr(part), part.stride(0), _lib.ptr(weight.data),
+                      _lib.ptr(weight.scale), weight.code, n, k, rows, _lib.EPI_ARGMAX, None, 0,
+                      None, 0, _lib.ptr(tokens[s:]), _lib.ptr(scratch), _lib.stream(x.device))
+        return tokens
     for s, e in _chunks(x.shape[0]):
         _launch(x[s:e], weight, weight.shape[0], _lib.EPI_ARGMAX, gain, eps,
                 tokens=tokens[s:e])

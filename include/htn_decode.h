@@ -260,6 +260,36 @@ int htn_gemm_tiles(const void* x, int64_t x_stride, const void* w, int64_t n, in
  * The two orders of the fp32 sums may round an output 1 bf16 ulp apart. */
 int64_t htn_gemm_tiles_scratch_bytes(int64_t rows, int64_t n, int64_t k, int epilogue);
 
+/* htn_gemm_tiles over 8-bit weights: w holds one byte per weight (weight_format
+ * HTN_WEIGHT_INT8 or HTN_WEIGHT_FP8_E4M3) and w_scale one float per weight row
+ * (2n for SwiGLU), multiplied into the fp32 sum as htn_gemv_w8 does; any number
+ * of rows. HTN_EPI_ARGMAX (at most HTN_GEMM_TILES_ARGMAX_ROWS rows) writes
+ * tokens[rows] instead of y. y of any stride and alignment. scratch:
+ * htn_gemm_tiles_w8_scratch_bytes bytes, 16-byte aligned; NULL, where the
+ * epilogue is not the argmax, keeps every tile's k range whole.
+ * The reference decodes in bf16 only; the row counts are those of its verify
+ * pass and prefill (decode.py:156-179). */
+#define HTN_GEMM_TILES_ARGMAX_ROWS 32
+int64_t htn_gemm_tiles_w8_scratch_bytes(int64_t rows, int64_t n, int64_t k, int epilogue,
+                                        int weight_format);
+int htn_gemm_tiles_w8(const void* x, int64_t x_stride, const void* w, const float* w_scale,
+                      int weight_format, int64_t n, int64_t k, int64_t rows, int epilogue,
+                      const void* residual, int64_t res_stride, void* y, int64_t y_stride,
+                      int64_t* tokens, void* scratch, htn_stream_t stream);
+
+/* The residual projection of htn_gemm_tiles (weight_format 0, w_scale unused)
+ * or htn_gemm_tiles_w8, and normed[m, :n] = rms_norm(y[m]) with `gain`: in the
+ * k split's finish when the tiles split k, else one launch more; the same bits
+ * either way. scratch as the HTN_EPI_RESIDUAL projection's
+ * (htn_gemm_tiles_w8_scratch_bytes; NULL: k whole).
+ * Replaces the reference's split_down_residual_norm
+ * (dryft/engine/kernels/split_down.py:85-101) over a prompt's rows. */
+int htn_gemm_tiles_residual_norm(const void* x, int64_t x_stride, const void* w,
+                                 const float* w_scale, int weight_format, int64_t n, int64_t k,
+                                 int64_t rows, const void* residual, int64_t res_stride, void* y,
+                                 int64_t y_stride, const void* gain, float eps, void* normed,
+                                 void* scratch, htn_stream_t stream);
+
 /* y[m, n] = bf16(sum_k x[m, k] * w[n, k]) (fp32 accumulation) for every row
  * m < rows, through hipBLASLt: the plain product of a prefill projection,
  * whose epilogues (residual add with the next RMSNorm, SwiGLU) then run as
