@@ -334,6 +334,7 @@ struct AttnArgs {
   int B, Hq, Hkv, G, Q, splits, split, stream;
   int ring;             // LDS-staged kernel: tiles staged ahead (0: other kernels)
   int mfma;             // LDS-staged kernel: tiles on the matrix cores
+  int pf_turn;          // attention_prefill_long: query ranks from here on run in reverse
   float scale;
   unsigned* done;       // arrival counters: XCD-affine grid, in-kernel merge (else null)
   // Blocks from attn_blocks on read the next projection's weights (pf_units
@@ -2184,18 +2185,25 @@ __device__ __forceinline__ void wait_v32(u32x2_t (&w)[4][8]) {
                : "memory");
 }
 
+__device__ __forceinline__ void wait_v16(u32x2_t (&w)[2][8]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[0][2]), "+v"(w[0][3]), "+v"(w[0][4]),
+                 "+v"(w[0][5]), "+v"(w[0][6]), "+v"(w[0][7]), "+v"(w[1][0]), "+v"(w[1][1]),
+                 "+v"(w[1][2]), "+v"(w[1][3]), "+v"(w[1][4]), "+v"(w[1][5]), "+v"(w[1][6]),
+                 "+v"(w[1][7])
+               :
+               : "memory");
+}
+
 constexpr int kPfQ = 64;                          // queries per prefill block
 constexpr int kPfTileBytes = 2 * kSplit * D * 2;  // K then V of one staged 64-slot tile
 
 // Causal attention over many queries per sequence (a prompt's prefill): one
 // launch per layer, no split, no merge. Block = (64-query tile, query head h,
-// batch b), four waves of 16 queries, or HPB = 2 query heads of one kv head
-// (eight waves: the second head's waves 4-7) sharing each staged tile. The
-// block stages each 64-slot K/V tile of kv head h / G once for its waves
-// (four waves a quarter each, LDS-direct, K and V, or with eight waves K by
-// waves 0-3 and V by 4-7; the next tile in flight), then every wave
-// multiplies all 64 slots against
-// its queries on the matrix cores as the decode kernel does per 16-slot
+// batch b), four waves of 16 queries. The block stages each 64-slot K/V tile
+// of kv head h / G once for its waves (a quarter each, LDS-direct, K and V; the
+// next tile in flight), then every wave multiplies all 64 slots against its
+// queries on the matrix cores as the decode kernel does per 16-slot
 // group: S^T = K Q^T (slots as M, queries as N: four 16-slot M-tiles x four
 // 32-dim steps), an online softmax per query in base 2, O^T += V^T P^T with P
 // as hi/lo bf16 halves (weights keep ~16 bits; the denominator sums the fp32
@@ -2204,20 +2212,18 @@ constexpr int kPfTileBytes = 2 * kSplit * D * 2;  // K then V of one staged 64-s
 // first. K rows are staged rotated (chunk c of slot s at column (c + s) % 16)
 // and V rows by two chunks per slot (c + 2 (s % 8)); V^T operands come from
 // transpose reads, one per 16 dims and 16 slots.
-template <int HPB>
-__global__ __launch_bounds__(HPB * kBlock) void attention_prefill(AttnArgs a) {
+__global__ __launch_bounds__(kBlock) void attention_prefill(AttnArgs a) {
   preload_args<false>(a);
-  constexpr int NW = HPB * kBlock / kWave;  // waves: HPB heads x four 16-query groups
+  constexpr int NW = kBlock / kWave;
   extern __shared__ __align__(16) unsigned char ring[];  // two staged tiles
   __shared__ int wave_pos[NW];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int qw = wave & 3;  // this wave's 16 queries of the block's 64
   const int col = lane & 15, quad = lane >> 4;
   const int ntq = (a.Q + kPfQ - 1) / kPfQ;
   const int qt = ntq - 1 - static_cast<int>(blockIdx.x);  // latest queries first
-  const int h = blockIdx.y * HPB + (wave >> 2), b = blockIdx.z, kvh = h / a.G;
-  const int t = qt * kPfQ + qw * 16 + col;  // this lane's query
+  const int h = blockIdx.y, b = blockIdx.z, kvh = h / a.G;
+  const int t = qt * kPfQ + wave * 16 + col;  // this lane's query
   const int tq = t < a.Q ? t : a.Q - 1;
   // Visible slots [0, pos]; a position past the cache sees every slot, a
   // negative one (and a padding query) none.
@@ -2253,22 +2259,16 @@ __global__ __launch_bounds__(HPB * kBlock) void attention_prefill(AttnArgs a) {
     kvoff[u] = static_cast<uint32_t>(sl * 256 + (((lane & 15) - sl) & 15) * 16);
     vvoff[u] = static_cast<uint32_t>(sl * 256 + (((lane & 15) - 2 * (sl & 7)) & 15) * 16);
   }
-  // With two heads per block (eight waves), waves 0-3 stage the K rows and
-  // waves 4-7 the V rows of their 16 slots.
   auto stage = [&](int kt) {
-    unsigned char* tb = ring + (kt & 1) * kPfTileBytes + qw * 4096;
-    const uint32_t off = static_cast<uint32_t>(kt * kSplit + qw * 16) * D * 2;
-    if (HPB == 1 || wave < 4) {
+    unsigned char* tb = ring + (kt & 1) * kPfTileBytes + wave * 4096;
+    const uint32_t off = static_cast<uint32_t>(kt * kSplit + wave * 16) * D * 2;
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void_t*)(tb + u * 1024), 16, kvoff[u], off, 0, 0);
-    }
-    if (HPB == 1 || wave >= 4) {
+    for (int u = 0; u < 4; ++u)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void_t*)(tb + u * 1024), 16, kvoff[u], off, 0, 0);
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void_t*)(tb + kSplit * D * 2 + u * 1024), 16,
-                                                 vvoff[u], off, 0, 0);
-    }
+    for (int u = 0; u < 4; ++u)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void_t*)(tb + kSplit * D * 2 + u * 1024), 16,
+                                               vvoff[u], off, 0, 0);
   };
   if (nkt > 0) stage(0);
 
@@ -2399,6 +2399,232 @@ __global__ __launch_bounds__(HPB * kBlock) void attention_prefill(AttnArgs a) {
     for (int j = 0; j < 8; ++j)
       *reinterpret_cast<uint2*>(dst + 16 * j) =
           make_uint2(pack_bf2(acc[j][0] / ln, acc[j][1] / ln), pack_bf2(acc[j][2] / ln, acc[j][3] / ln));
+  }
+}
+
+// Causal attention over long prompts: as attention_prefill, but every wave
+// takes 32 queries (two 16-query N tiles), so each K and V^T operand read from
+// LDS feeds two products. Block = four waves: HPB query heads of one kv head
+// (2, or 1 for an odd group) x 64 / 128 queries sharing each staged tile; two
+// blocks per CU, whose waves overlap one's softmax with the other's products.
+//
+// bit-identical to attention_prefill (the same tiles, products and sums per
+// query). Per layer, 32 query heads on 8 kv heads: 1500 queries 72 -> 56 us,
+// 2048 126 -> 72, 5000 497 -> 305 (672 TFLOP/s counted once, 1.5 times that on
+// the matrix cores, since the weights multiply as two halves); 4 sequences of
+// 512 39 -> 25. What bounds it: per wave and tile 96 products (1536 cycles)
+// and some 370 vector instructions with 32 exponentials (1900 cycles), which
+// two waves per SIMD (242 registers) hardly overlap: raising the priority of
+// either phase, or interleaving one group's products with the next one's
+// weights, measured the same or slower (5000 queries: 302, 330 us).
+template <int HPB>
+__global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(AttnArgs a) {
+  preload_args<false>(a);
+  constexpr int QW = 4 / HPB;       // 32-query groups per head
+  constexpr int BQ = 32 * QW;       // queries per block
+  extern __shared__ __align__(16) unsigned char ring[];  // two staged tiles
+  __shared__ int wave_pos[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, quad = lane >> 4;
+  // Block L takes head unit L % units (units of one kv head a multiple of Hkv
+  // apart: on one XCD where Hkv is a multiple of 8) and query rank L / units.
+  // Ranks run from the latest queries, the longest, to the first; where every
+  // block is resident at once (two per CU), the second half runs the other
+  // way, so that a CU's two blocks sum to the same work.
+  const int units = a.B * a.Hq / HPB, ntq = (a.Q + BQ - 1) / BQ;
+  const int u = static_cast<int>(blockIdx.x) % units;
+  int rank = static_cast<int>(blockIdx.x) / units;
+  if (rank >= a.pf_turn) rank = ntq - 1 - (rank - a.pf_turn);
+  const int qt = ntq - 1 - rank;
+  const int b = u / (a.Hq / HPB), hu = u % (a.Hq / HPB);
+  const int kvh = hu % a.Hkv;
+  const int h = kvh * a.G + (hu / a.Hkv) * HPB + wave / QW;
+  const int t0 = qt * BQ + (wave % QW) * 32 + col;  // this lane's queries: t0, t0 + 16
+  // Visible slots [0, pos]; a position past the cache sees every slot, a
+  // negative one (and a padding query) none.
+  int pos[2];
+  u32x4 qf[2][4];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const int t = t0 + 16 * n, tq = t < a.Q ? t : a.Q - 1;
+    const int64_t pv = a.pos[tq];
+    pos[n] = t >= a.Q || pv < 0 ? -1 : (pv >= a.cap ? static_cast<int>(a.cap) - 1 : static_cast<int>(pv));
+    // B operand of S^T = K Q^T: dims 32 ks + 8 quad .. + 7 of the query.
+    const bf16_t* qrow = a.q + b * a.q_sb + h * a.q_sh + tq * a.q_st + 8 * quad;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[n][ks] = *reinterpret_cast<const u32x4*>(qrow + 32 * ks);
+  }
+  const float wmax = wave_max(static_cast<float>(pos[0] > pos[1] ? pos[0] : pos[1]));  // exact: |pos| < 2^24
+  const float wmin = -wave_max(-static_cast<float>(pos[0] < pos[1] ? pos[0] : pos[1]));
+  if (lane == 0) wave_pos[wave] = static_cast<int>(wmax);
+  lds_barrier();
+  int bmax = wave_pos[0];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) bmax = wave_pos[w] > bmax ? wave_pos[w] : bmax;
+  const int nkt = bmax < 0 ? 0 : bmax / kSplit + 1;  // tiles [0, nkt) hold every visible slot
+  const int wave_last = static_cast<int>(wmax), wave_first = static_cast<int>(wmin);
+
+  // Staging and operand addresses as attention_prefill's four-wave block.
+  const long kv_base = (static_cast<long>(b) * a.Hkv + kvh) * a.cap * D;
+  const uint32_t range = static_cast<uint32_t>(bmax + 1) * D * 2;  // block-uniform (from LDS)
+  const __amdgpu_buffer_rsrc_t krs = uniform_rsrc(a.keys + kv_base, range);
+  const __amdgpu_buffer_rsrc_t vrs = uniform_rsrc(a.values + kv_base, range);
+  uint32_t kvoff[4], vvoff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int sl = 4 * i + (lane >> 4);
+    kvoff[i] = static_cast<uint32_t>(sl * 256 + (((lane & 15) - sl) & 15) * 16);
+    vvoff[i] = static_cast<uint32_t>(sl * 256 + (((lane & 15) - 2 * (sl & 7)) & 15) * 16);
+  }
+  auto stage = [&](int kt) {
+    unsigned char* tb = ring + (kt & 1) * kPfTileBytes + wave * 4096;
+    const uint32_t off = static_cast<uint32_t>(kt * kSplit + wave * 16) * D * 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void_t*)(tb + i * 1024), 16, kvoff[i], off, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void_t*)(tb + kSplit * D * 2 + i * 1024), 16,
+                                               vvoff[i], off, 0, 0);
+  };
+  if (nkt > 0) stage(0);
+
+  const uint32_t ring_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)ring));
+  uint32_t kaddr[4], vaddr[8];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    kaddr[ks] = ring_base + static_cast<uint32_t>(col * 256 + (((4 * ks + quad + col) & 15) * 16));
+  const int vr = 4 * quad + (col >> 2);
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    vaddr[j] = ring_base + kSplit * D * 2 +
+               static_cast<uint32_t>(vr * 256 + (((2 * j + ((col & 3) >> 1) + 2 * (vr & 7)) & 15) * 16) +
+                                     (col & 1) * 8);
+
+  const float scale2 = a.scale * 1.4426950408889634f;  // log2(e) / sqrt(D)
+  f32x4_t acc[2][8];
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[n][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int kt = 0; kt < nkt; ++kt) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (kt + 1 < nkt) stage(kt + 1);
+    const int s0 = kt * kSplit;
+    if (s0 > wave_last) continue;  // wave-uniform: no slot of the tile is visible to the wave
+    const uint32_t tb = static_cast<uint32_t>((kt & 1) * kPfTileBytes);
+    u32x4 kf[4][4];
+    issue_k_pf<0>(kaddr[0] + tb, kf[0]);
+    issue_k_pf<0>(kaddr[1] + tb, kf[1]);
+    issue_k_pf<0>(kaddr[2] + tb, kf[2]);
+    issue_k_pf<0>(kaddr[3] + tb, kf[3]);
+    wait_k16(kf);
+    f32x4_t st[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) st[n][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+          st[n][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8_t, kf[ks][mt]), __builtin_bit_cast(bf16x8_t, qf[n][ks]),
+              st[n][mt], 0, 0, 0);
+    // The V^T operands of half the tile in flight during the softmax.
+    uint32_t va[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) va[j] = vaddr[j] + tb;
+    u32x2_t vw[2][8];
+    issue_vt_tr<0>(va, vw[0]);
+    issue_vt_tr<4096>(va, vw[1]);
+    uint4 phl[2][4];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      float sc[4][4];
+      float tmax = -INFINITY;
+      if (__builtin_expect(s0 + kSplit - 1 <= wave_first, 1)) {
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            sc[mt][i] = st[n][mt][i] * scale2;
+            tmax = fmaxf(tmax, sc[mt][i]);
+          }
+      } else {
+        const int lim = pos[n] - s0 - 4 * quad;  // slot s0 + 16 mt + 4 quad + i visible iff 16 mt + i <= lim
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float v = st[n][mt][i] * scale2;
+            sc[mt][i] = 16 * mt + i <= lim ? v : -INFINITY;
+            tmax = fmaxf(tmax, sc[mt][i]);
+          }
+      }
+      tmax = quad_max(tmax);
+      const float m_new = fmaxf(m[n], tmax);
+      // A query with nothing visible yet keeps weight 0 (no inf - inf).
+      const float ms = m_new == -INFINITY ? 0.f : m_new;
+      if (!__all(m_new == m[n])) {
+        const float alpha = __builtin_amdgcn_exp2f(m[n] - ms);  // 0 while m is -inf
+        l[n] *= alpha;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[n][j] *= alpha;
+      }
+      m[n] = m_new;
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = __builtin_amdgcn_exp2f(sc[mt][i] - ms);
+        l[n] += (p[0] + p[1]) + (p[2] + p[3]);
+        const uint2 pb = make_uint2(pack_bf2(p[0], p[1]), pack_bf2(p[2], p[3]));
+        const uint2 pl = make_uint2(pack_bf2(p[0] - bf_lo(pb.x), p[1] - bf_hi(pb.x)),
+                                    pack_bf2(p[2] - bf_lo(pb.y), p[3] - bf_hi(pb.y)));
+        phl[n][mt] = make_uint4(pb.x, pb.y, pl.x, pl.y);
+      }
+    }
+    auto weigh = [&](const u32x2_t (&v2)[2][8], int mt0) {
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const u32x4 v = {v2[mt][j].x, v2[mt][j].y, v2[mt][j].x, v2[mt][j].y};
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+            acc[n][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8_t, v), __builtin_bit_cast(bf16x8_t, phl[n][mt0 + mt]),
+                acc[n][j], 0, 0, 0);
+        }
+    };
+    wait_v16(vw);
+    u32x2_t vx[2][8];
+    issue_vt_tr<8192>(va, vx[0]);
+    issue_vt_tr<12288>(va, vx[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    weigh(vw, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_v16(vx);
+    weigh(vx, 2);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // O[query][dim 16 j + 4 quad + i] = acc[j][i] / (the four quads' sums).
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    const float ln = quad_sum(l[n]);
+    const int t = t0 + 16 * n;
+    if (t >= a.Q) continue;
+    bf16_t* dst = a.out + b * a.o_sb + h * a.o_sh + static_cast<long>(t) * a.o_st + 4 * quad;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      *reinterpret_cast<uint2*>(dst + 16 * j) =
+          make_uint2(pack_bf2(acc[n][j][0] / ln, acc[n][j][1] / ln), pack_bf2(acc[n][j][2] / ln, acc[n][j][3] / ln));
   }
 }
 
@@ -2699,6 +2925,17 @@ constexpr long kPrefetchXcdBytes = 3L << 20;
 // two per XCD outlast the attention, 2.44 ms).
 constexpr int kPrefetchPerXcdLong = 4;
 
+template <int HPB>
+int launch_prefill_long(const AttnArgs& a, long blocks, size_t lds, hipStream_t st) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&attention_prefill_long<HPB>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  (void)attr;  // a refused size surfaces as a launch error
+  hipLaunchKernelGGL(attention_prefill_long<HPB>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock),
+                     lds, st, a);
+  return launch_status();
+}
+
 // Many queries per sequence (a prefill): the causal kernel, one launch, no
 // scratch. Needs 16-byte query fragments and 8-byte output stores.
 int run_prefill_attention(AttnArgs& a, hipStream_t st) {
@@ -2710,26 +2947,24 @@ int run_prefill_attention(AttnArgs& a, hipStream_t st) {
     return HTN_EUNSUPPORTED;
   a.scale = 1.0f / sqrtf(static_cast<float>(D));
   const size_t lds = 2 * static_cast<size_t>(kPfTileBytes);
-  static const hipError_t attr1 = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&attention_prefill<1>), hipFuncAttributeMaxDynamicSharedMemorySize,
+  // Long prompts: two heads of a kv head (one, for an odd group) per block
+  // with 32 queries per wave, as soon as its blocks outnumber the CUs (8B,
+  // 1024 queries, 256 blocks: 38 us either way; 1500 72 -> 56; 512 16.5 -> 21).
+  const int hpb = a.G % 2 == 0 ? 2 : 1;
+  const long units = static_cast<long>(a.B) * a.Hq / hpb;
+  const long bq = 128 / hpb, nq = (a.Q + bq - 1) / bq, cus = device_cus();
+  if (units * nq > cus && units * nq * hpb < (1L << 31)) {
+    a.pf_turn = static_cast<int>(units * nq <= 2 * cus ? (cus + units - 1) / units : nq);
+    return hpb == 2 ? launch_prefill_long<2>(a, units * nq, lds, st)
+                    : launch_prefill_long<1>(a, units * nq, lds, st);
+  }
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&attention_prefill), hipFuncAttributeMaxDynamicSharedMemorySize,
       static_cast<int>(lds));
-  static const hipError_t attr2 = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&attention_prefill<2>), hipFuncAttributeMaxDynamicSharedMemorySize,
-      static_cast<int>(lds));
-  (void)attr1;  // a refused size surfaces as a launch error
-  (void)attr2;
-  // Two query heads of one kv head per block share each staged tile while
-  // the grid keeps two blocks per CU (8B, 2048 queries: 151 -> 146 us; at
-  // 512 queries the halved grid measured slower, 18.6 -> 23.0 us).
-  const long ntq = (a.Q + kPfQ - 1) / kPfQ;
-  const int hpb =
-      a.G % 2 == 0 && ntq * (a.Hq / 2) * a.B >= 2L * device_cus() ? 2 : 1;
-  const dim3 grid(static_cast<unsigned>(ntq), static_cast<unsigned>(a.Hq / hpb),
+  (void)attr;  // a refused size surfaces as a launch error
+  const dim3 grid(static_cast<unsigned>((a.Q + kPfQ - 1) / kPfQ), static_cast<unsigned>(a.Hq),
                   static_cast<unsigned>(a.B));
-  if (hpb == 2)
-    hipLaunchKernelGGL(attention_prefill<2>, grid, dim3(2 * kBlock), lds, st, a);
-  else
-    hipLaunchKernelGGL(attention_prefill<1>, grid, dim3(kBlock), lds, st, a);
+  hipLaunchKernelGGL(attention_prefill, grid, dim3(kBlock), lds, st, a);
   return launch_status();
 }
 

@@ -1,0 +1,48 @@
+"""Causal attention over long prompts: the 32-query kernel against the 16-query one.
+
+A query's result depends on its own row, position and the cache alone, so the
+whole prompt in one call (more blocks than CUs: the long kernel) must equal,
+bit for bit, the same queries in calls of a few rows (the short kernel), which
+the oracle tests cover.
+"""
+import pytest
+import torch
+
+from hackthenorth_amd.kernels.attention import grouped_attention
+
+pytestmark = pytest.mark.gpu
+
+# (batch, heads, kv heads, queries, first position): one and four sequences, a
+# ragged last tile, odd group sizes (one head per block), eight heads on one kv
+# head, and just past one and past two blocks per CU (the order of the query
+# tiles turns between them).
+CASES = [(1, 32, 8, 1089, 0), (1, 32, 8, 2113, 0), (4, 32, 8, 300, 37), (1, 24, 8, 1500, 0),
+         (1, 32, 32, 1100, 5), (2, 16, 8, 1111, 100), (1, 8, 1, 4200, 0), (3, 32, 8, 500, 700)]
+
+
+@pytest.mark.parametrize("order", ["causal", "shuffled"])
+@pytest.mark.parametrize("batch,heads,kv_heads,queries,first", CASES)
+def test_long_prompt_equals_short_calls(batch, heads, kv_heads, queries, first, order):
+    g = torch.Generator(device="cuda").manual_seed(queries)
+    capacity = first + queries + 9
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+    q = normal(batch, queries, heads, 128).transpose(1, 2)
+    k, v = normal(batch, kv_heads, capacity, 128), normal(batch, kv_heads, capacity, 128)
+    k[:, :, first + queries:] = float("nan")  # unwritten slots stay unread
+    v[:, :, first + queries:] = float("nan")
+    positions = first + torch.arange(queries, device="cuda")
+    if order == "shuffled":
+        positions = positions[torch.randperm(queries, generator=g, device="cuda")]
+    whole = torch.empty(batch, queries, heads, 128, dtype=torch.bfloat16,
+                        device="cuda").transpose(1, 2)
+    grouped_attention(q, k, v, positions, out=whole)
+    step = 64
+    for b in range(batch):
+        for s in range(0, queries, step):
+            part = q[b:b + 1, :, s:s + step]
+            if part.shape[2] <= 8:  # a verify pass's rows: another kernel
+                continue
+            short = grouped_attention(part, k[b:b + 1], v[b:b + 1], positions[s:s + step])
+            assert torch.equal(whole[b:b + 1, :, s:s + step], short)
