@@ -42,6 +42,13 @@ constexpr int kMaxRowsMT = 128; // eight 16-row tiles (prefill chunks, large bat
 constexpr int kMaxRowsI = 32;   // rows per launch of the interleaved gate/up kernel
 constexpr int kU = 1;          // k steps per wave per batch (1 measured fastest of 1, 2, 4)
 constexpr int kMaxWaves = 16;
+// Weights of this size or more are streamed past the caches: a model that has
+// them has more of them than the last-level cache holds. 5 rows, weights from
+// HBM, 8B: O 9.4 -> 8.4 us, gate/up 39.6 -> 35.4, down 22.3 -> 19.8, head 227
+// -> 200 (6.2 TB/s); 4B: 7.9 -> 7.4, 25.0 -> 23.8, 14.7 -> 14.2, 144 -> 130.
+// The 0.6B's smaller ones, where they stay cached from one pass to the next,
+// lose (O 4.3 -> 4.8, down 4.9 -> 5.7).
+constexpr long kStreamBytes = 16L << 20;
 constexpr int kMaxK = 16384;
 
 struct RowsArgs {
@@ -101,7 +108,8 @@ constexpr int kPitch = 144;  // bytes per staged 64-element weight row (+16: con
 // across the first weight issue (82-92 VGPRs unbounded: 5 waves per SIMD);
 // bounded to 8 (S = 1, 60 VGPRs) and 6 (S = 2, 80) waves per SIMD without
 // spills (8B 16-row batched step 3634 -> 3657 tok/s, 5-row verify unchanged).
-template <int MT, int S, int EPI, int W, bool NORM>
+// AUX: the weight loads' cache policy, 2 (non-temporal) past kStreamBytes.
+template <int MT, int S, int EPI, int W, bool NORM, int AUX>
 __global__ __launch_bounds__(W * 64, NORM && MT == 1 ? (S == 1 ? 8 : 6) : 1) void gemm_rows_kernel(RowsArgs a) {
   preload_rows(a);
   if constexpr (NORM) asm volatile("" ::"s"(a.xgain), "s"(a.xeps));
@@ -153,8 +161,8 @@ __global__ __launch_bounds__(W * 64, NORM && MT == 1 ? (S == 1 ? 8 : 6) : 1) voi
       const uint32_t soff = static_cast<uint32_t>(j < j1 ? j : 0) * kStep * 2u;           \
       _Pragma("unroll") for (int s = 0; s < S; ++s) {                                     \
         const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(sbase[s], range);                   \
-        wv[u][s][0] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff0, soff, 0);         \
-        wv[u][s][1] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff1, soff, 0);         \
+        wv[u][s][0] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff0, soff, AUX);       \
+        wv[u][s][1] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff1, soff, AUX);       \
       }                                                                                   \
     }                                                                                     \
   }
@@ -582,8 +590,12 @@ int choose_splits(int strips, int waves, int K) {
 template <int MT, int S, int EPI, int W, bool NORM>
 int launch_w(RowsArgs& a, hipStream_t st) {
   const int strips = (a.N + kStrip - 1) / kStrip;
-  hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM>), dim3(strips, a.KS), dim3(W * 64), 0,
-                     st, a);
+  if (2L * S * a.N * a.K >= kStreamBytes)
+    hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, 2>), dim3(strips, a.KS), dim3(W * 64),
+                       0, st, a);
+  else
+    hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, 0>), dim3(strips, a.KS), dim3(W * 64),
+                       0, st, a);
   if (launch_status() != HTN_OK) return HTN_ELAUNCH;
   if (EPI == HTN_EPI_ARGMAX) {
     hipLaunchKernelGGL(gemm_rows_argmax, dim3(a.M), dim3(kBlock), 0, st, a.keys, strips, a.M, a.tokens);
