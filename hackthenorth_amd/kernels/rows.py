@@ -3,7 +3,7 @@
 The speculative verify pass scores k + 1 tokens in one forward; the reference
 runs its multi-row projections as Triton GEMM tiles (dryft/engine/
 projections.py:168-183, kernels/gateup.py:40-58, kernels/split_down.py:85-101).
-Here up to STRIP_ROWS rows are one htn_gemm_rows launch (16-column strips, the
+Here few rows (STRIP_ROWS) are one htn_gemm_rows launch (16-column strips, the
 RMSNorm inside, plus a K-split reduction when the strips alone cannot fill the
 GPU) and more rows one htn_gemm_tiles launch (LDS-staged output tiles, plus the
 finish of its k split), with the batch-one GEMVs' bf16 rounding boundaries.
@@ -20,12 +20,15 @@ from ..quant import QuantizedWeight
 from .greedy import greedy_head
 
 MAX_ROWS = 128    # rows per htn_gemm_rows launch
-# Rows up to which bf16 projections take the strips: at 16 rows of the 8B
-# shape strips / tiles take 15.6 / 13.9 us for QKV and 18 / 15 for O without
-# their norms, which the strips compute inside (a launch, 4 us), and at 5 rows
-# of the 4B the strips win outright (8.9 / 10.4, 12.2 / 13.2); at 32 rows of
-# the 8B QKV, O, gate/up and down take 21 / 15, 21 / 15, 44 / 35 and 40 / 30.
-STRIP_ROWS = 16
+# Rows up to which bf16 projections take the strips, for weights of at least /
+# below LARGE elements. At 16 rows of the 8B shape strips / tiles take 19.6 /
+# 13.3 us for QKV, 9.5 / 13.2 for O, 40 / 35 for gate/up and 26 / 26 for down,
+# with the RMSNorm in the strips' QKV and gate/up and in the tiles' O and down;
+# at 5 rows 15 / 13, 8 / 12, 35 / 34 and 19 / 25; 4B, 16 rows, 15 / 11, 10 / 11,
+# 29 / 21 and 19 / 15. The 0.6B's weights fill too few tiles: at 8 rows 5 / 8,
+# 5 / 10, 6 / 8 and 5 / 11, at 32 rows 9 / 8, 7 / 10, 10 / 8 and 9 / 11.
+STRIP_ROWS, SMALL_STRIP_ROWS = 8, 32
+LARGE = 8 << 20
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
 # Rows from which a plain store (QKV) and a residual projection leave the
@@ -143,13 +146,14 @@ def _tiles_residual_norm(x, weight, residual, gain, eps):
 
 def tiled(x, weight):
     """Whether a projection of these rows takes the tiles: 8-bit weights
-    always, bf16 ones past STRIP_ROWS rows whose output rows the tiles' 8-byte
+    always, bf16 ones past the strips' rows whose output rows the tiles' 8-byte
     stores and whose input strides their 32-bit offsets cover (TILE_ROWS rows
     or more have no other kernel)."""
     if isinstance(weight, QuantizedWeight):
         return True
     rows = x.shape[0]
-    return rows >= TILE_ROWS or (rows > STRIP_ROWS and weight.shape[0] % 8 == 0
+    strips = STRIP_ROWS if weight.numel() >= LARGE else SMALL_STRIP_ROWS
+    return rows >= TILE_ROWS or (rows > strips and weight.shape[0] % 8 == 0
                                  and x.stride(0) < 1 << 22)
 
 
