@@ -57,7 +57,7 @@ struct RowsArgs {
   const bf16_t* res; long res_rs;
   bf16_t* y; long y_rs;
   float* part;          // [KS][M][Nw] fp32 (KS > 1)
-  uint64_t* keys;       // argmax: [strips][M]
+  uint64_t* keys;       // argmax: [M][strips]
   int64_t* tokens;      // argmax: [M]
   int M, N, K, KS, steps_per_split;
   // Residual epilogue fused with the next RMSNorm (K-split finish only):
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(W * 64, NORM && MT == 1 ? (S == 1 ? 8 : 6) : 1) voi
     if (tid < a.M) {
       uint64_t b = best[tid][0];
       for (int c = 1; c < kStrip; ++c) b = best[tid][c] > b ? best[tid][c] : b;
-      a.keys[static_cast<long>(strip) * a.M + tid] = b;
+      a.keys[static_cast<long>(tid) * gridDim.x + strip] = b;
     }
   }
 }
@@ -428,23 +428,34 @@ __global__ __launch_bounds__(kBlock) void gemm_rows_finish_norm(RowsArgs a) {
   }
 }
 
-// Per-row argmax over the strips' keys.
-__global__ __launch_bounds__(kBlock) void gemm_rows_argmax(const uint64_t* __restrict__ keys,
-                                                          int strips, int M, int64_t* tokens) {
-  asm volatile("" ::"s"(keys), "s"(strips), "s"(M), "s"(tokens));
-  __shared__ uint64_t wbest[4];
+// Per-row argmax over the strips' keys, a block of sixteen waves per row, eight
+// keys per thread in flight: one chain of loads per row, not its bytes, is the
+// time (5 rows of 9496 strips, 8B: the head 200 -> 193 us whole).
+constexpr int kArgmaxThreads = 1024;
+__global__ __launch_bounds__(kArgmaxThreads) void gemm_rows_argmax(const uint64_t* __restrict__ keys,
+                                                                   int strips, int64_t* tokens) {
+  asm volatile("" ::"s"(keys), "s"(strips), "s"(tokens));
+  __shared__ uint64_t wbest[kArgmaxThreads / kWave];
   const int m = blockIdx.x;
-  uint64_t b = 0;
-  for (int i = threadIdx.x; i < strips; i += kBlock) {
-    const uint64_t k = keys[static_cast<long>(i) * M + m];
-    b = k > b ? k : b;
+  const uint64_t* row = keys + static_cast<long>(m) * strips;
+  uint64_t b = 0;  // below every key
+  for (int i0 = threadIdx.x; i0 < strips; i0 += 8 * kArgmaxThreads) {
+    uint64_t k[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + u * kArgmaxThreads;
+      k[u] = row[i < strips ? i : i0];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b = k[u] > b ? k[u] : b;
   }
   b = wave_max_u64(b);
   if ((threadIdx.x & 63) == 0) wbest[threadIdx.x >> 6] = b;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t r = wbest[0];
-    for (int i = 1; i < 4; ++i) r = wbest[i] > r ? wbest[i] : r;
+#pragma unroll
+    for (int i = 1; i < kArgmaxThreads / kWave; ++i) r = wbest[i] > r ? wbest[i] : r;
     tokens[m] = static_cast<int64_t>(argmax_key_index(r));
   }
 }
@@ -598,7 +609,8 @@ int launch_w(RowsArgs& a, hipStream_t st) {
                        0, st, a);
   if (launch_status() != HTN_OK) return HTN_ELAUNCH;
   if (EPI == HTN_EPI_ARGMAX) {
-    hipLaunchKernelGGL(gemm_rows_argmax, dim3(a.M), dim3(kBlock), 0, st, a.keys, strips, a.M, a.tokens);
+    hipLaunchKernelGGL(gemm_rows_argmax, dim3(a.M), dim3(kArgmaxThreads), 0, st, a.keys, strips,
+                       a.tokens);
   } else if (a.KS > 1 && EPI == HTN_EPI_RESIDUAL && a.normed) {
     hipLaunchKernelGGL(gemm_rows_finish_norm, dim3(a.M), dim3(kBlock), 0, st, a);
   } else if (a.KS > 1) {
