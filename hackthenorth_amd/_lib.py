@@ -139,11 +139,21 @@ def call(name, *args):
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    """A tensor's address for a pointer argument (None: NULL). A plain integer:
+    a ctypes object per argument costs more than the call itself needs."""
+    return t.data_ptr() if t is not None else None
 
 
 def stream(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle on `device` (default: the current device).
+    The raw handle, without the Stream object torch.cuda.current_stream wraps
+    it in (an eager one-row add_rms_norm: 10.9 -> 8.6 us a call with this and `ptr`)."""
+    if device is not None and not isinstance(device, torch.device):
+        device = torch.device(device)
+    index = None if device is None else device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def require_gpu(*tensors):
