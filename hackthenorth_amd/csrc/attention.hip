@@ -331,10 +331,11 @@ struct AttnArgs {
   long o_sb, o_sh, o_st;
   float* part;          // [B, Hq, Q, splits, D]
   float* ml;            // [B, Hq, Q, splits, 2]
+  // split: slots per split; in attention_prefill_long, which has none, the
+  // query rank from which ranks run in reverse.
   int B, Hq, Hkv, G, Q, splits, split, stream;
   int ring;             // LDS-staged kernel: tiles staged ahead (0: other kernels)
   int mfma;             // LDS-staged kernel: tiles on the matrix cores
-  int pf_turn;          // attention_prefill_long: query ranks from here on run in reverse
   float scale;
   unsigned* done;       // arrival counters: XCD-affine grid, in-kernel merge (else null)
   // Blocks from attn_blocks on read the next projection's weights (pf_units
@@ -2435,7 +2436,7 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(AttnArgs a) 
   const int units = a.B * a.Hq / HPB, ntq = (a.Q + BQ - 1) / BQ;
   const int u = static_cast<int>(blockIdx.x) % units;
   int rank = static_cast<int>(blockIdx.x) / units;
-  if (rank >= a.pf_turn) rank = ntq - 1 - (rank - a.pf_turn);
+  if (rank >= a.split) rank = ntq - 1 - (rank - a.split);
   const int qt = ntq - 1 - rank;
   const int b = u / (a.Hq / HPB), hu = u % (a.Hq / HPB);
   const int kvh = hu % a.Hkv;
@@ -2954,7 +2955,7 @@ int run_prefill_attention(AttnArgs& a, hipStream_t st) {
   const long units = static_cast<long>(a.B) * a.Hq / hpb;
   const long bq = 128 / hpb, nq = (a.Q + bq - 1) / bq, cus = device_cus();
   if (units * nq > cus && units * nq * hpb < (1L << 31)) {
-    a.pf_turn = static_cast<int>(units * nq <= 2 * cus ? (cus + units - 1) / units : nq);
+    a.split = static_cast<int>(units * nq <= 2 * cus ? (cus + units - 1) / units : nq);
     return hpb == 2 ? launch_prefill_long<2>(a, units * nq, lds, st)
                     : launch_prefill_long<1>(a, units * nq, lds, st);
   }
