@@ -27,7 +27,7 @@
 //  * SwiGLU tiles interleave gate and up rows in groups of 16 (32 with 2 x 2
 //    waves), so a lane holds the gate and up dot products of the same outputs;
 //  * when the tiles leave block slots empty, each tile's k range splits over
-//    up to 8 blocks; they store fp32 partial sums and a second launch adds
+//    up to 12 blocks; they store fp32 partial sums and a second launch adds
 //    them in split order and applies the epilogue (with the next RMSNorm, when
 //    the caller wants it);
 //  * blocks are laid out XCD-major: the blocks of one weight tile share an
@@ -591,8 +591,9 @@ constexpr TileShape kShapes[] = {
 
 // A launch's time by those coefficients: per XCD, `blocks` blocks of `steps`
 // k steps in rounds of two per CU (one, for eight waves), no less than the
-// weights take from HBM, the launch itself, and for a k split its finish: a launch, the partial sums' bytes, and for
-// the finish with a norm (a block per row) its chain over the splits.
+// weights take from HBM, the launch itself, and for a k split its finish: a
+// launch, the partial sums' bytes, and for the finish with a norm (a block per
+// row) its chain over the splits.
 float tile_cost(const TileShape& sh, long blocks, long steps, long ks, double part_mb,
                 double weight_mb, bool residual, int format) {
   const long cus = device_cus() / 8 > 0 ? device_cus() / 8 : 1;

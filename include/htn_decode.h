@@ -237,7 +237,8 @@ int htn_gemm_rows_residual_norm(const void* x, int64_t x_stride, const void* w, 
 
 /* The projection of many rows at once (a prompt's prefill: hundreds to
  * thousands of rows): y = x W^T as a tiled GEMM on the matrix cores, one
- * launch, 128 x 128 output tiles, both operands staged in LDS (weight tiles
+ * launch, output tiles of 16 to 256 rows x 128 or 256 columns chosen by size,
+ * both operands staged in LDS (weight tiles
  * reused from the L2 of one XCD by every row tile). Epilogues HTN_EPI_STORE,
  * HTN_EPI_RESIDUAL and HTN_EPI_SWIGLU as htn_gemm_rows (w holds 2n rows for
  * SwiGLU: gate rows, then up rows); no input RMSNorm (normalise the rows
@@ -253,8 +254,8 @@ int htn_gemm_tiles(const void* x, int64_t x_stride, const void* w, int64_t n, in
                    int64_t y_stride, void* scratch, htn_stream_t stream);
 
 /* Scratch bytes htn_gemm_tiles uses for these sizes (0: none). When the tile
- * grid alone fills at most half of the blocks the CUs hold at once (prompts
- * of a few hundred rows), each tile's k range splits over up to 8 blocks whose fp32
+ * grid alone leaves block slots empty (few rows, long k; never a bf16 grid of
+ * 128 x 128 tiles that fills them), each tile's k range splits over up to 12 blocks whose fp32
  * partial sums go to `scratch` (16-byte aligned) and a second launch adds
  * them in split order; with scratch NULL every tile sums its whole k range.
  * The two orders of the fp32 sums may round an output 1 bf16 ulp apart. */

@@ -18,11 +18,13 @@ pytestmark = pytest.mark.gpu
 FORMATS = ["bf16", "int8", "fp8_e4m3"]
 # Rows around the tiles' edges (16 to 256 rows), widths off the 128- and
 # 256-row weight tiles and off the eight XCD columns, k of one step, of fewer
-# steps than the staging ring and of several splits.
+# steps than the staging ring and of several splits; the last seven take the
+# 128- and 160-row tiles and the eight-wave ones of 128 to 256 rows.
 CASES = [(2, 40, 64), (16, 136, 192), (17, 1000, 2560), (33, 136, 512), (48, 264, 1024),
          (49, 2568, 576), (65, 1032, 4096), (97, 520, 2048), (129, 2560, 1088),
          (160, 264, 9728), (201, 1544, 1024), (225, 5128, 640), (300, 6144, 1024),
-         (513, 2560, 2048)]
+         (513, 2560, 2048), (160, 12296, 512), (225, 12296, 640), (300, 12296, 640),
+         (450, 8200, 1024), (500, 12288, 512), (700, 6152, 640), (1000, 6152, 640)]
 
 
 def bf16(seed, *shape, std=1.0):
@@ -42,10 +44,11 @@ def weight(fmt, n, k, seed):
 
 
 def check_store(got, x, values):
-    exact = x.double() @ values.T
-    slack = x.shape[1] * 2.0 ** -24 * (x.double().abs() @ values.abs().T)
+    x, values = x.double().cuda(), values.cuda()
+    exact = x @ values.T
+    slack = x.shape[1] * 2.0 ** -24 * (x.abs() @ values.abs().T)
     ulp = torch.pow(2.0, torch.floor(torch.log2(exact.abs().clamp_min(1e-30))) - 7)
-    assert bool(((got.cpu().double() - exact).abs() <= ulp + slack).all())
+    assert bool(((got.double() - exact).abs() <= ulp + slack).all())
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
@@ -58,10 +61,11 @@ def test_tiles_match_the_exact_product(fmt, m, n, k):
     check_store(RW._tiles(xd, half, n, RW._lib.EPI_STORE), x, values[:n])
     res, gain = bf16(3, m, n), bf16(4, n)
     out, normed = RW._tiles_residual_norm(xd, half, res.cuda(), gain.cuda(), 1e-6)
-    y = (x.double() @ values.T).to(torch.bfloat16)
+    y = (x.double().cuda() @ values.cuda().T).to(torch.bfloat16).cpu()
     torch.testing.assert_close(out.cpu().float(), (y[:, :n].float() + res.float()),
                                atol=2e-2, rtol=2e-2)
-    assert torch.equal(normed, rms_norm(out, gain.cuda(), 1e-6))
+    if n <= 8192:  # the standalone norm takes rows of up to 8192 columns
+        assert torch.equal(normed, rms_norm(out, gain.cuda(), 1e-6))
     gu = y.float()
     torch.testing.assert_close(RW._tiles(xd, w, n, RW._lib.EPI_SWIGLU).cpu().float(),
                                torch.nn.functional.silu(gu[:, :n]) * gu[:, n:],
@@ -109,3 +113,15 @@ def test_tiles_replay_in_a_graph(fmt):
             torch.cuda.synchronize()
             assert torch.equal(out[0], eager[0]) and torch.equal(out[1], eager[1])
             RW._tiles_residual_norm(x, w, res, gain, 1e-6)
+
+
+@pytest.mark.parametrize("m,v", [(2, 16), (3, 2000), (5, 16400), (8, 150000)])
+def test_strip_argmax_over_few_and_many_strips(m, v):
+    """The strips' per-row finish: one strip, under and over 1024 strips (one
+    key per thread), over 8192 (a thread's second round)."""
+    x, w = bf16(11, m, 64).cuda(), bf16(12, v, 64).cuda()
+    got = RW.greedy_rows(x, w)
+    logits = x.double() @ w.double().T
+    best = logits.max(dim=1).values
+    ulp = torch.pow(2.0, torch.floor(torch.log2(best.abs())) - 7)
+    assert bool((best - logits.gather(1, got[:, None])[:, 0] <= ulp).all())
