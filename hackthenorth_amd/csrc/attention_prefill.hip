@@ -8,6 +8,8 @@
 // 4B fp8 decode slice at 30 K slots took 268.2 us in place of 265.9.
 #include "attention.h"
 
+#include <type_traits>
+
 namespace htn {
 
 // The kernel arguments read before the first vector load, named as scalar
@@ -297,21 +299,30 @@ __global__ __launch_bounds__(kBlock) void attention_prefill(PrefillArgs a) {
   }
 }
 
+template <typename T>
+__device__ __forceinline__ void swap(T& a, T& b) {
+  const T t = a;
+  a = b;
+  b = t;
+}
+
 // Causal attention over long prompts: as attention_prefill, but every wave
 // takes 32 queries (two 16-query N tiles), so each K and V^T operand read from
 // LDS feeds two products. Block = four waves: HPB query heads of one kv head
 // (2, or 1 for an odd group) x 64 / 128 queries sharing each staged tile; two
 // blocks per CU, whose waves overlap one's softmax with the other's products.
 //
-// bit-identical to attention_prefill (the same tiles, products and sums per
-// query). Per layer, 32 query heads on 8 kv heads: 1500 queries 72 -> 56 us,
-// 2048 126 -> 72, 5000 497 -> 305 (672 TFLOP/s counted once, 1.5 times that on
-// the matrix cores, since the weights multiply as two halves); 4 sequences of
-// 512 39 -> 25. What bounds it: per wave and tile 96 products (1536 cycles)
-// and some 370 vector instructions with 32 exponentials (1900 cycles), which
-// two waves per SIMD (242 registers) hardly overlap: raising the priority of
-// either phase, or interleaving one group's products with the next one's
-// weights, measured the same or slower (5000 queries: 302, 330 us).
+// Bit-identical to attention_prefill (the same tiles, products and sums per
+// query), also where V holds infinities or NaN: of a tile, a query weighs the
+// slots that its 16-query group and its 64-query tile reach there. Per layer,
+// 32 query heads on 8 kv heads: 1500 queries 72 -> 56 us, 2048 126 -> 72, 5000
+// 497 -> 305 (672 TFLOP/s counted once, 1.5 times that on the matrix cores,
+// since the weights multiply as two halves); 4 sequences of 512 39 -> 25. What
+// bounds it: per wave and tile 96 products (1536 cycles) and some 370 vector
+// instructions with 32 exponentials (1900 cycles), which two waves per SIMD
+// (244 registers) hardly overlap: raising the priority of either phase, or
+// interleaving one group's products with the next one's weights, measured the
+// same or slower (5000 queries: 302, 330 us).
 template <int HPB>
 __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs a) {
   preload_prefill(a);
@@ -350,15 +361,22 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) qf[n][ks] = *reinterpret_cast<const u32x4*>(qrow + 32 * ks);
   }
-  const float wmax = wave_max(static_cast<float>(pos[0] > pos[1] ? pos[0] : pos[1]));  // exact: |pos| < 2^24
-  const float wmin = -wave_max(-static_cast<float>(pos[0] < pos[1] ? pos[0] : pos[1]));
-  if (lane == 0) wave_pos[wave] = static_cast<int>(wmax);
+  // The last slot each 16-query group of the wave sees (exact: |pos| < 2^24).
+  auto wave_top = [](int v) {
+    return __builtin_amdgcn_readfirstlane(static_cast<int>(wave_max(static_cast<float>(v))));
+  };
+  const int last0 = wave_top(pos[0]), last1 = wave_top(pos[1]);
+  const int wave_first = -wave_top(pos[0] < pos[1] ? -pos[0] : -pos[1]);
+  if (lane == 0) wave_pos[wave] = last0 > last1 ? last0 : last1;
   lds_barrier();
   int bmax = wave_pos[0];
 #pragma unroll
   for (int w = 1; w < 4; ++w) bmax = wave_pos[w] > bmax ? wave_pos[w] : bmax;
   const int nkt = bmax < 0 ? 0 : bmax / kSplit + 1;  // tiles [0, nkt) hold every visible slot
-  const int wave_last = static_cast<int>(wmax), wave_first = static_cast<int>(wmin);
+  // The last slot that the 64 queries around the wave's see: with one head per
+  // block, the other 64 may see more of a tile.
+  const int near = __builtin_amdgcn_readfirstlane(
+      wave_pos[wave & 2] > wave_pos[wave | 1] ? wave_pos[wave & 2] : wave_pos[wave | 1]);
 
   // Staging and operand addresses as attention_prefill's four-wave block.
   const long kv_base = (static_cast<long>(b) * a.Hkv + kvh) * a.cap * D;
@@ -404,12 +422,10 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
   for (int n = 0; n < 2; ++n)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[n][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int kt = 0; kt < nkt; ++kt) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
-    if (kt + 1 < nkt) stage(kt + 1);
+  // The work of one tile for the wave's groups N0 and 1.
+  auto tile = [&](int kt, auto n0) {
+    constexpr int N0 = decltype(n0)::value;
     const int s0 = kt * kSplit;
-    if (s0 > wave_last) continue;  // wave-uniform: no slot of the tile is visible to the wave
     const uint32_t tb = static_cast<uint32_t>((kt & 1) * kPfTileBytes);
     u32x4 kf[4][4];
     issue_k_pf<0>(kaddr[0] + tb, kf[0]);
@@ -419,11 +435,11 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
     wait_k16(kf);
     f32x4_t st[2][4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+    for (int n = N0; n < 2; ++n)
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) st[n][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
+    for (int n = N0; n < 2; ++n)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -440,7 +456,7 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
     issue_vt_tr<4096>(va, vw[1]);
     uint4 phl[2][4];
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
+    for (int n = N0; n < 2; ++n) {
       float sc[4][4];
       float tmax = -INFINITY;
       if (__builtin_expect(s0 + kSplit - 1 <= wave_first, 1)) {
@@ -487,16 +503,26 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
     }
     auto weigh = [&](const u32x2_t (&v2)[2][8], int mt0) {
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
+      for (int mt = 0; mt < 2; ++mt) {
+        // With one head per block, slots past `near` as zeros: the lane's
+        // slots are 0 .. e of the four from s0 + 16 (mt0 + mt) + 4 quad.
+        uint32_t lo = ~0u, hi = ~0u;
+        if constexpr (HPB == 1 && N0 == 1) {
+          const int e = near - s0 - 16 * (mt0 + mt) - 4 * quad;
+          lo = e < 0 ? 0u : (e == 0 ? 0xffffu : ~0u);
+          hi = e < 2 ? 0u : (e == 2 ? 0xffffu : ~0u);
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const u32x4 v = {v2[mt][j].x, v2[mt][j].y, v2[mt][j].x, v2[mt][j].y};
+          const uint32_t x = v2[mt][j].x & lo, y = v2[mt][j].y & hi;
+          const u32x4 v = {x, y, x, y};
 #pragma unroll
-          for (int n = 0; n < 2; ++n)
+          for (int n = N0; n < 2; ++n)
             acc[n][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 __builtin_bit_cast(bf16x8_t, v), __builtin_bit_cast(bf16x8_t, phl[n][mt0 + mt]),
                 acc[n][j], 0, 0, 0);
         }
+      }
     };
     wait_v16(vw);
     u32x2_t vx[2][8];
@@ -507,6 +533,37 @@ __global__ __launch_bounds__(kBlock, 2) void attention_prefill_long(PrefillArgs 
     __builtin_amdgcn_sched_barrier(0);
     wait_v16(vx);
     weigh(vx, 2);
+  };
+  auto next_tile = [&](int kt) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (kt + 1 < nkt) stage(kt + 1);
+  };
+  // A weight of zero times an infinite or NaN V is NaN, so a group takes part
+  // in the tiles it sees a slot of and no others, and weighs no slot past
+  // `near`: first the tiles that both groups see and that end by `near`, both
+  // groups at once, then the few others one group at a time, as group 1. Every
+  // wave passes nkt barriers, wherever its two loops part.
+  const int first_last = last0 < last1 ? last0 : last1;
+  int whole = first_last < 0 ? 0 : first_last / kSplit + 1;
+  if (HPB == 1 && whole > (near + 1) / kSplit) whole = (near + 1) / kSplit;
+  for (int kt = 0; kt < whole; ++kt) {
+    next_tile(kt);
+    tile(kt, std::integral_constant<int, 0>{});
+  }
+  for (int kt = whole; kt < nkt; ++kt) {
+    next_tile(kt);
+#pragma unroll 1
+    for (int g = 1; g >= 0; --g) {
+      if (kt * kSplit <= (g == 1 ? last1 : last0)) tile(kt, std::integral_constant<int, 1>{});
+#pragma unroll
+      for (int j = 0; j < 8; ++j) swap(acc[0][j], acc[1][j]);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) swap(qf[0][ks], qf[1][ks]);
+      swap(pos[0], pos[1]);
+      swap(m[0], m[1]);
+      swap(l[0], l[1]);
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // O[query][dim 16 j + 4 quad + i] = acc[j][i] / (the four quads' sums).

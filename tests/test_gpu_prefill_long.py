@@ -46,3 +46,40 @@ def test_long_prompt_equals_short_calls(batch, heads, kv_heads, queries, first, 
                 continue
             short = grouped_attention(part, k[b:b + 1], v[b:b + 1], positions[s:s + step])
             assert torch.equal(whole[b:b + 1, :, s:s + step], short)
+
+
+# (batch, heads, kv heads, queries, first position): first positions at which a
+# wave's two 16-query groups, and with one head per block (odd groups) a block's
+# two 64-query halves, end in different 64-slot tiles.
+NONFINITE_CASES = [(4, 32, 8, 300, 37), (2, 16, 8, 1111, 100), (1, 32, 8, 1500, 48),
+                   (1, 24, 8, 1500, 40), (1, 32, 32, 1100, 5), (16, 24, 8, 200, 93)]
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("order", ["causal", "shuffled"])
+@pytest.mark.parametrize("batch,heads,kv_heads,queries,first", NONFINITE_CASES)
+def test_later_nonfinite_values_reach_no_further_than_in_short_calls(batch, heads, kv_heads,
+                                                                     queries, first, order, value):
+    """One infinite or NaN V per kv head, at slots that the earlier half of the
+    queries does not see: what is finite in short calls is finite, and the same."""
+    g = torch.Generator(device="cuda").manual_seed(queries)
+    capacity = first + queries + 9
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+    q = normal(batch, queries, heads, 128).transpose(1, 2)
+    k, v = normal(batch, kv_heads, capacity, 128), normal(batch, kv_heads, capacity, 128)
+    tile = 64 * -(-(first + queries // 2) // 64)
+    for j in range(kv_heads):
+        v[:, j, min(tile + 7 * j % 64, first + queries - 1), 3 * j] = value
+    positions = first + torch.arange(queries, device="cuda")
+    if order == "shuffled":
+        positions = positions[torch.randperm(queries, generator=g, device="cuda")]
+    whole = grouped_attention(q, k, v, positions)
+    for s in range(0, queries, 64):
+        part = q[:1, :, s:s + 64]
+        if part.shape[2] > 8:
+            short = grouped_attention(part, k[:1], v[:1], positions[s:s + 64])
+            torch.testing.assert_close(whole[:1, :, s:s + 64], short, rtol=0, atol=0,
+                                       equal_nan=True)
+    assert bool(whole.isfinite().any())
