@@ -607,10 +607,15 @@ int prefill_attention(PrefillArgs& a, hipStream_t st) {
   // Long prompts: two heads of a kv head (one, for an odd group) per block
   // with 32 queries per wave, as soon as its blocks outnumber the CUs (8B,
   // 1024 queries, 256 blocks: 38 us either way; 1500 72 -> 56; 512 16.5 -> 21).
+  // One head's blocks hold 128 queries, twice the short kernel's: they take
+  // grids that they pad by at most a tenth more (24 heads on 8 kv heads, 16
+  // sequences of 64 queries 8.2 us short, 10.7 long; 4 of 300 15.5 / 17.6; 4 of
+  // 512 33 / 25; 2 of 700 31 / 29).
   const int hpb = a.G % 2 == 0 ? 2 : 1;
   const long units = static_cast<long>(a.B) * a.Hq / hpb;
   const long bq = 128 / hpb, nq = (a.Q + bq - 1) / bq, cus = device_cus();
-  if (units * nq > cus && units * nq * hpb < (1L << 31)) {
+  const long padded = bq * nq, padded_short = (a.Q + kPfQ - 1) / kPfQ * kPfQ;
+  if (units * nq > cus && units * nq * hpb < (1L << 31) && 10 * padded <= 11 * padded_short) {
     a.turn = static_cast<int>(units * nq <= 2 * cus ? (cus + units - 1) / units : nq);
     return hpb == 2 ? launch_prefill_long<2>(a, units * nq, lds, st)
                     : launch_prefill_long<1>(a, units * nq, lds, st);
