@@ -147,14 +147,15 @@ def _tiles_residual_norm(x, weight, residual, gain, eps):
 def tiled(x, weight):
     """Whether a projection of these rows takes the tiles: 8-bit weights
     always, bf16 ones past the strips' rows whose output rows the tiles' 8-byte
-    stores and whose input strides their 32-bit offsets cover (TILE_ROWS rows
-    or more have no other kernel)."""
+    stores and whose input strides their 32-bit offsets cover, unless the input
+    rows overlap (an expanded row, sliding windows: the strips read those);
+    TILE_ROWS rows or more have no other kernel."""
     if isinstance(weight, QuantizedWeight):
         return True
     rows = x.shape[0]
     strips = STRIP_ROWS if weight.numel() >= LARGE else SMALL_STRIP_ROWS
     return rows >= TILE_ROWS or (rows > strips and weight.shape[0] % 8 == 0
-                                 and x.stride(0) < 1 << 22)
+                                 and x.shape[1] <= x.stride(0) < 1 << 22)
 
 
 def _scratch(device, rows, n, k, epilogue, norm):

@@ -1,0 +1,57 @@
+"""Which kernel the multi-row projections take for rows of unusual strides:
+what the strips accept is not sent to the tiles, which refuse it. The routes are looked up on the CPU, the results compared on the GPU."""
+import pytest
+import torch
+
+from hackthenorth_amd.kernels import rows as RW
+
+
+def matrix(rows, cols, layout, device="cpu", seed=0):
+    """bf16 [rows, cols]: contiguous, padded rows, one row expanded, or windows
+    that slide by eight elements."""
+    g = torch.Generator().manual_seed(seed)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(device)
+    if layout == "expanded":
+        return normal(1, cols).expand(rows, cols)
+    if layout == "windows":
+        return normal(8 * rows + cols).as_strided((rows, cols), (8, 1))
+    if layout == "padded":
+        return normal(rows, cols + 24)[:, :cols]
+    return normal(rows, cols)
+
+
+@pytest.mark.parametrize("rows,n,k", [(9, 4096, 4096), (33, 512, 1024), (100, 512, 1024),
+                                      (255, 4096, 4096)])
+def test_overlapping_rows_stay_on_the_strips(rows, n, k):
+    w = torch.empty(n, k, dtype=torch.bfloat16)
+    assert not RW.tiled(matrix(rows, k, "expanded"), w)
+    assert not RW.tiled(matrix(rows, k, "windows"), w)
+    assert RW.tiled(matrix(rows, k, "padded"), w) == RW.tiled(matrix(rows, k, "plain"), w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["expanded", "windows", "padded"])
+@pytest.mark.parametrize("rows,n,k", [(9, 4096, 2048), (20, 4096, 2048), (40, 264, 1024),
+                                      (129, 512, 9728), (255, 1000, 512)])
+def test_rows_of_any_stride_give_the_contiguous_rows_results(rows, n, k, layout):
+    x = matrix(rows, k, layout, "cuda")
+    w = 0.02 * matrix(2 * n, k, "plain", "cuda", 1)
+    top, res = w[:n].contiguous(), matrix(rows, n, "plain", "cuda", 2)
+    gain = matrix(1, n, "plain", "cuda", 3)[0]
+    xg = matrix(1, k, "plain", "cuda", 4)[0]
+    y = x.float() @ top.float().T
+    kw = dict(atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(RW.projection_rows(x, top).float(), y, **kw)
+    if rows <= 32 or layout == "padded":  # the row-wise norm reads no overlapping rows
+        torch.testing.assert_close(RW.projection_rows(x, top, xg).float(),
+                                   RW.projection_rows(x.contiguous(), top, xg).float(), **kw)
+    out, normed = RW.residual_norm_rows(x, top, res, gain)
+    torch.testing.assert_close(out.float(), y.bfloat16().float() + res.float(), **kw)
+    torch.testing.assert_close(RW.residual_rows(x, top, res).float(), out.float(), **kw)
+    torch.testing.assert_close(normed.float(), torch.nn.functional.rms_norm(
+        out.float(), (n,), gain.float(), 1e-6), **kw)
+    gu = (x.float() @ w.float().T).bfloat16().float()
+    torch.testing.assert_close(RW.swiglu_rows(x, w).float(),
+                               torch.nn.functional.silu(gu[:, :n]) * gu[:, n:], **kw)
