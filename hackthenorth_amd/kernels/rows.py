@@ -158,6 +158,18 @@ def tiled(x, weight):
                                  and x.shape[1] <= x.stride(0) < 1 << 22)
 
 
+def norm_tiled(x, weight, residual):
+    """Whether a residual projection with the next RMSNorm takes the tiles: of
+    a prompt's rows up to LIBRARY_ROWS, and there not those of which the
+    library's product and the row-wise residual add take more: widths off the
+    64-wide k steps, residual rows that overlap, far strides."""
+    if not prompt(x, weight):
+        return tiled(x, weight)
+    n, k = weight.shape
+    return x.shape[0] <= LIBRARY_ROWS and k % 64 == 0 and residual.stride(0) >= n \
+        and x.stride(0) < 1 << 22
+
+
 def _scratch(device, rows, n, k, epilogue, norm):
     nbytes = _lib.load().htn_gemm_rows_scratch_bytes(rows, n, k, epilogue, int(norm))
     if nbytes <= 0:
@@ -241,7 +253,7 @@ def residual_norm_rows(x, weight, residual, gain, eps=1e-6):
             or not gain.is_contiguous():
         raise ValueError("gain must be a contiguous bf16 [N] vector")
     _lib.require_gpu(x, _weight(weight)[0], residual, gain)
-    if tiled(x, weight) and not (prompt(x, weight) and x.shape[0] > LIBRARY_ROWS):
+    if norm_tiled(x, weight, residual):
         return _tiles_residual_norm(x, weight, residual, gain, eps)
     if x.shape[0] >= TILE_ROWS:
         rows = x.shape[0]

@@ -1,5 +1,6 @@
-"""Which kernel the multi-row projections take for rows of unusual strides:
-what the strips accept is not sent to the tiles, which refuse it. The routes are looked up on the CPU, the results compared on the GPU."""
+"""Which kernel the multi-row projections take for rows of unusual strides and
+widths: what the strips and the library accept is not sent to the tiles, which
+refuse it. The routes are looked up on the CPU, the results compared on the GPU."""
 import pytest
 import torch
 
@@ -31,6 +32,18 @@ def test_overlapping_rows_stay_on_the_strips(rows, n, k):
     assert RW.tiled(matrix(rows, k, "padded"), w) == RW.tiled(matrix(rows, k, "plain"), w)
 
 
+@pytest.mark.parametrize("rows", [256, 300, 512])
+def test_residual_norm_of_a_prompt_leaves_what_the_tiles_refuse_to_the_library(rows):
+    n, k = 512, 1024
+    w, res = torch.empty(n, k, dtype=torch.bfloat16), matrix(rows, n, "plain")
+    x = matrix(rows, k, "plain")
+    assert RW.norm_tiled(x, w, res) and RW.norm_tiled(matrix(rows, k, "padded"), w, res)
+    assert not RW.norm_tiled(x, w, matrix(rows, n, "expanded"))
+    for off in (8, 40):  # the library takes every multiple of eight
+        assert not RW.norm_tiled(matrix(rows, k + off, "plain"),
+                                 torch.empty(n, k + off, dtype=torch.bfloat16), res)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["expanded", "windows", "padded"])
 @pytest.mark.parametrize("rows,n,k", [(9, 4096, 2048), (20, 4096, 2048), (40, 264, 1024),
@@ -55,3 +68,16 @@ def test_rows_of_any_stride_give_the_contiguous_rows_results(rows, n, k, layout)
     gu = (x.float() @ w.float().T).bfloat16().float()
     torch.testing.assert_close(RW.swiglu_rows(x, w).float(),
                                torch.nn.functional.silu(gu[:, :n]) * gu[:, n:], **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k,layout", [(256, 512, 1032, "plain"), (512, 264, 520, "plain"),
+                                             (300, 512, 1024, "expanded")])
+def test_residual_norm_rows_off_the_tiles(rows, n, k, layout):
+    x, w = matrix(rows, k, "plain", "cuda"), 0.02 * matrix(n, k, "plain", "cuda", 1)
+    res, gain = matrix(rows, n, layout, "cuda", 2), matrix(1, n, "plain", "cuda", 3)[0]
+    out, normed = RW.residual_norm_rows(x, w, res, gain)
+    torch.testing.assert_close(out.float(), (x.float() @ w.float().T).bfloat16().float() + res.float(),
+                               atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(normed.float(), torch.nn.functional.rms_norm(
+        out.float(), (n,), gain.float(), 1e-6), atol=2e-2, rtol=2e-2)
