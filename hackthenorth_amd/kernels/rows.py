@@ -20,15 +20,19 @@ from ..quant import QuantizedWeight
 from .greedy import greedy_head
 
 MAX_ROWS = 128    # rows per htn_gemm_rows launch
-# Rows up to which bf16 projections take the strips, for weights of at least /
-# below LARGE elements. At 16 rows of the 8B shape strips / tiles take 19.6 /
-# 13.3 us for QKV, 9.5 / 13.2 for O, 40 / 35 for gate/up and 26 / 26 for down,
-# with the RMSNorm in the strips' QKV and gate/up and in the tiles' O and down;
-# at 5 rows 15 / 13, 8 / 12, 35 / 34 and 19 / 25; 4B, 16 rows, 15 / 11, 10 / 11,
-# 29 / 21 and 19 / 15. The 0.6B's weights fill too few tiles: at 8 rows 5 / 8,
-# 5 / 10, 6 / 8 and 5 / 11, at 32 rows 9 / 8, 7 / 10, 10 / 8 and 9 / 11.
-STRIP_ROWS, SMALL_STRIP_ROWS = 8, 32
-LARGE = 8 << 20
+# Rows up to which bf16 projections take the strips: of weights of at least
+# LARGE elements, of those whose shorter side is at least WIDE too, and of
+# smaller ones. Strips / tiles, in us, with the RMSNorm in the strips' QKV and
+# gate/up and in the tiles' O and down:
+#   8B, QKV, O, gate/up, down: 9 rows 16, 9, 34, 20 / 14, 14, 32, 29; 16 rows 20,
+#   10, 38, 24 / 15, 14, 32, 31 (a slice of the model: 432 / 482 and 486 / 496);
+#   17 rows, two row tiles per strip, 23, 11, 41, 26 / 15, 14, 33, 30;
+#   4B: 9 rows 12, 8, 24, 14 / 11, 11, 21, 16; 16 rows 15, 9, 28, 18 / 12, 11,
+#   21, 17 (O and down are 160 strips of 16 columns, too few for the CUs; from
+#   4096 columns on there is a strip per CU);
+#   0.6B: 8 rows 5, 5, 6, 5 / 8, 10, 8, 11; 32 rows 9, 7, 10, 9 / 8, 10, 8, 11.
+STRIP_ROWS, WIDE_STRIP_ROWS, SMALL_STRIP_ROWS = 8, 16, 32
+LARGE, WIDE = 8 << 20, 4096
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
 # Rows from which a plain store (QKV) and a residual projection leave the
@@ -153,7 +157,8 @@ def tiled(x, weight):
     if isinstance(weight, QuantizedWeight):
         return True
     rows = x.shape[0]
-    strips = STRIP_ROWS if weight.numel() >= LARGE else SMALL_STRIP_ROWS
+    strips = SMALL_STRIP_ROWS if weight.numel() < LARGE \
+        else WIDE_STRIP_ROWS if min(weight.shape) >= WIDE else STRIP_ROWS
     return rows >= TILE_ROWS or (rows > strips and weight.shape[0] % 8 == 0
                                  and x.shape[1] <= x.stride(0) < 1 << 22)
 

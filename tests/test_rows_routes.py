@@ -23,7 +23,17 @@ def matrix(rows, cols, layout, device="cpu", seed=0):
     return normal(rows, cols)
 
 
-@pytest.mark.parametrize("rows,n,k", [(9, 4096, 4096), (33, 512, 1024), (100, 512, 1024),
+@pytest.mark.parametrize("n,k,strips", [(1024, 2048, 32), (2560, 9728, 8), (6144, 2560, 8),
+                                        (4096, 12288, 16), (24576, 4096, 16)])
+def test_strips_end_by_weight_size(n, k, strips):
+    """The last row count on the strips: small weights, large ones, and large ones
+    with at least a strip of 16 columns per CU in every projection of the model."""
+    w = torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+    for rows in (strips, strips + 1):
+        assert RW.tiled(torch.empty(rows, k, device="meta"), w) == (rows > strips)
+
+
+@pytest.mark.parametrize("rows,n,k", [(17, 4096, 4096), (33, 512, 1024), (100, 512, 1024),
                                       (255, 4096, 4096)])
 def test_overlapping_rows_stay_on_the_strips(rows, n, k):
     w = torch.empty(n, k, dtype=torch.bfloat16)
