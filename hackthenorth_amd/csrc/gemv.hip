@@ -418,7 +418,10 @@ constexpr long kWavesPerCu = 16;
 // takes 9.9 us at two, 10.6 us at four, and three, two rows per wave, made
 // the 8B step 2.831 -> 2.847 ms); 8-bit rows are half as long, so a
 // wave holds half the bytes in flight: their norm kernels keep four blocks
-// per CU (eight for 1 KB rows).
+// per CU (eight for 1 KB rows). Greedy heads count their blocks alike without
+// the norm, since a block leaves a key for the finish to read (16882 rows, bf16
+// / int8: K = 2560 23.7 -> 20.6 / 17.8 -> 16.6 us, K = 4096 27.6 -> 25.8 /
+// 19.6 -> 18.7; 151936 rows, K = 2560 135 -> 130 / 99 either way).
 long blocks_per_cu(long groups, bool norm, int epi, int wf, long k) {
   if (wf == WF_BF16 && (epi == EPI_RESIDUAL ? !norm : (norm && epi == EPI_SWIGLU))) {
     const long want = epi == EPI_RESIDUAL ? 2 : 3;
@@ -426,7 +429,7 @@ long blocks_per_cu(long groups, bool norm, int epi, int wf, long k) {
     for (long pc = 1; pc <= 8; pc *= 2)
       if (groups == pc * 4 * cus * want) return pc;
   }
-  if (norm) return wf == WF_BF16 ? 2 : (k > 1024 ? 4 : 8);
+  if (norm || epi == EPI_ARGMAX) return wf == WF_BF16 ? 2 : (k > 1024 ? 4 : 8);
   return 8;
 }
 

@@ -33,6 +33,11 @@ MAX_ROWS = 128    # rows per htn_gemm_rows launch
 #   0.6B: 8 rows 5, 5, 6, 5 / 8, 10, 8, 11; 32 rows 9, 7, 10, 9 / 8, 10, 8, 11.
 STRIP_ROWS, WIDE_STRIP_ROWS, SMALL_STRIP_ROWS = 8, 16, 32
 LARGE, WIDE = 8 << 20, 4096
+# Bytes from which a bf16 vocabulary is streamed past the caches, one row of it
+# as the batch-one head (a smaller one is still cached from the last pass: a
+# row without the norm 8.7 us on the strips, 10.6 on the head; 33 MB from HBM
+# 12.1 / 10.2).
+STREAM_HEAD_BYTES = 64 << 20
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
 # Rows from which a plain store (QKV) and a residual projection leave the
@@ -305,12 +310,18 @@ def swiglu_rows(x, gate_up_weight, gain=None, eps=1e-6):
     return out
 
 
+def streams_head(weight):
+    """Whether one row against this vocabulary takes the batch-one head without
+    a norm to share its launch: 8-bit ones and bf16 ones of STREAM_HEAD_BYTES."""
+    return isinstance(weight, QuantizedWeight) or 2 * weight.numel() >= STREAM_HEAD_BYTES
+
+
 def greedy_rows(x, weight, gain=None, eps=1e-6):
     """argmax_n bf16(W x_m) per row (lowest id on ties); gain applies RMSNorm first."""
     _check(x, weight)
     _lib.require_gpu(x, _weight(weight)[0], gain)
     tokens = torch.empty((x.shape[0],), dtype=torch.int64, device=x.device)
-    if x.shape[0] == 1 and x.is_contiguous():
+    if x.shape[0] == 1 and x.is_contiguous() and (gain is not None or streams_head(weight)):
         # The batch-one head normalises in its launch and streams the weight
         # with nothing else to do (8B: 182 us against 220).
         return greedy_head(x, gain, eps, weight, tokens)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from hackthenorth_amd.kernels import rows as RW
+from hackthenorth_amd.kernels.rmsnorm import rms_norm
 
 
 def matrix(rows, cols, layout, device="cpu", seed=0):
@@ -91,3 +92,28 @@ def test_residual_norm_rows_off_the_tiles(rows, n, k, layout):
                                atol=2e-2, rtol=2e-2)
     torch.testing.assert_close(normed.float(), torch.nn.functional.rms_norm(
         out.float(), (n,), gain.float(), 1e-6), atol=2e-2, rtol=2e-2)
+
+
+def test_small_vocabularies_keep_cached_loads():
+    def vocabulary(v, k):
+        return torch.empty(v, k, dtype=torch.bfloat16, device="meta")
+    assert not RW.streams_head(vocabulary(32767, 1024)) and RW.streams_head(vocabulary(32768, 1024))
+    codes, scale = torch.empty(16, 64, dtype=torch.uint8), torch.empty(16)
+    assert RW.streams_head(RW.QuantizedWeight(codes, scale, "int8"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [32767, 32768])  # either side of the streamed size
+@pytest.mark.parametrize("rows", [1, 3, 17, 40])
+def test_greedy_rows_around_the_streamed_size(vocab, rows):
+    x, w = matrix(rows, 1024, "plain", "cuda"), matrix(vocab, 1024, "plain", "cuda", 1)
+    gain = matrix(1, 1024, "plain", "cuda", 2)[0]
+    for g in (None, gain):
+        xn = x if g is None else rms_norm(x, g, 1e-6)
+        logits = xn.double() @ w.double().T
+        got, best = RW.greedy_rows(x, w, g), logits.max(dim=1).values
+        ulp = torch.pow(2.0, torch.floor(torch.log2(best)) - 7)
+        # In the head's launch, the norm's sum of squares in another order may round
+        # an element of a row the other way: four of the largest at most.
+        slack = 0 if g is None else 4 * 2.0 ** -8 * float(xn.abs().max()) * float(w.abs().max())
+        assert bool((best - logits.gather(1, got[:, None])[:, 0] <= ulp + slack).all())
