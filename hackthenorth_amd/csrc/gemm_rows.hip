@@ -49,6 +49,10 @@ constexpr int kMaxWaves = 16;
 // The 0.6B's smaller ones, where they stay cached from one pass to the next,
 // lose (O 4.3 -> 4.8, down 4.9 -> 5.7).
 constexpr long kStreamBytes = 16L << 20;
+// A vocabulary smaller than this belongs to a model that the last-level cache
+// holds between passes (33 MB of one, among 125 MB of weights: 8.1 us cached,
+// 9.0 streamed; alone at 86 MB 20.2 / 21.9, but from HBM 23.7 / 23.0).
+constexpr long kStreamHeadBytes = 64L << 20;
 constexpr int kMaxK = 16384;
 
 struct RowsArgs {
@@ -108,7 +112,8 @@ constexpr int kPitch = 144;  // bytes per staged 64-element weight row (+16: con
 // across the first weight issue (82-92 VGPRs unbounded: 5 waves per SIMD);
 // bounded to 8 (S = 1, 60 VGPRs) and 6 (S = 2, 80) waves per SIMD without
 // spills (8B 16-row batched step 3634 -> 3657 tok/s, 5-row verify unchanged).
-// AUX: the weight loads' cache policy, 2 (non-temporal) past kStreamBytes.
+// AUX: the weight loads' cache policy, 2 (non-temporal) from kStreamBytes
+// (kStreamHeadBytes) on.
 template <int MT, int S, int EPI, int W, bool NORM, int AUX>
 __global__ __launch_bounds__(W * 64, NORM && MT == 1 ? (S == 1 ? 8 : 6) : 1) void gemm_rows_kernel(RowsArgs a) {
   preload_rows(a);
@@ -601,7 +606,7 @@ int choose_splits(int strips, int waves, int K) {
 template <int MT, int S, int EPI, int W, bool NORM>
 int launch_w(RowsArgs& a, hipStream_t st) {
   const int strips = (a.N + kStrip - 1) / kStrip;
-  if (2L * S * a.N * a.K >= kStreamBytes)
+  if (2L * S * a.N * a.K >= (EPI == HTN_EPI_ARGMAX ? kStreamHeadBytes : kStreamBytes))
     hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, 2>), dim3(strips, a.KS), dim3(W * 64),
                        0, st, a);
   else
