@@ -84,6 +84,15 @@ struct TileArgs {
 // staging alone, 268 MB in 256 tiles: all from k = 0 4.4 TB/s, rotated 6.05,
 // rotated and past the caches (one row tile) 6.7.
 constexpr int kRotate = 37;
+// Weights of this size or more are streamed past the caches by the tiles of at
+// most 48 rows, and from kStreamOnceBytes on where a single row tile reads them.
+// From HBM streaming is faster: 4B int8, one tile, QKV of 15.7 MB 10.1 -> 9.3
+// us, O of 10.5 MB 11.4 -> 10.6; 8B at 32 rows in two tiles, O 15.0 -> 14.5,
+// down 35.7 -> 34.5. A small model's weights are still in the last-level cache
+// from the pass before (100 MB of them read in turn, 0.6B at 48 rows: QKV 6.4
+// cached / 8.2 streamed, gate/up of 12.6 MB 6.5 / 8.2; from HBM 8.3 / 8.0 and
+// 8.4 / 8.1).
+constexpr long kStreamBytes = 16L << 20, kStreamOnceBytes = 10L << 20;
 constexpr int kMinSplitSteps = 8;     // k steps each split keeps at least
 constexpr int kMaxSplit = 12;
 
@@ -239,13 +248,12 @@ __device__ __forceinline__ void stage_tiles(unsigned char* st, int ks, bool live
   }
 }
 
-template <int EPI, int WM, int WN, int NT, int WF>
+// AUX: the weight loads' cache policy (kStreamBytes).
+template <int EPI, int WM, int WN, int NT, int WF, int AUX>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tiles_kernel(TileArgs a) {
   using S = Shape<WM, WN, NT, WF>;
   constexpr bool SW = EPI == HTN_EPI_SWIGLU;
   constexpr int WT = S::kWt, TM = S::kTm;
-  // Weights of a single row tile are read once: streamed past the caches.
-  constexpr int AUX = WM == 1 ? 2 : 0;
   // Arguments in scalar registers at entry: one round of scalar loads.
   asm volatile("" ::"s"(a.x), "s"(a.x_rs), "s"(a.w), "s"(a.scale), "s"(a.res), "s"(a.res_rs),
                "s"(a.y), "s"(a.y_rs), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.mtiles), "s"(a.ntiles),
@@ -650,18 +658,29 @@ long tiles_scratch_bytes(const TilePlan& p, long rows) {
   return p.ksplit > 1 ? static_cast<long>(p.ksplit) * rows * p.part_rs * 4 : p.keys_bytes;
 }
 
-template <int EPI, int WM, int WN, int NT, int WF>
-int launch_shape(TileArgs& a, long blocks, hipStream_t st) {
+template <int EPI, int WM, int WN, int NT, int WF, int AUX>
+int launch_policy(const TileArgs& a, long blocks, hipStream_t st) {
   using S = Shape<WM, WN, NT, WF>;
   constexpr int bytes = S::kStages * S::kStage;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&gemm_tiles_kernel<EPI, WM, WN, NT, WF>),
+      reinterpret_cast<const void*>(&gemm_tiles_kernel<EPI, WM, WN, NT, WF, AUX>),
       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   (void)attr;  // a refused size surfaces as a launch error
-  a.mtiles = (a.M + S::kTm - 1) / S::kTm;
-  hipLaunchKernelGGL((gemm_tiles_kernel<EPI, WM, WN, NT, WF>), dim3(static_cast<unsigned>(blocks)),
-                     dim3(64 * S::kWaves), bytes, st, a);
+  hipLaunchKernelGGL((gemm_tiles_kernel<EPI, WM, WN, NT, WF, AUX>),
+                     dim3(static_cast<unsigned>(blocks)), dim3(64 * S::kWaves), bytes, st, a);
   return launch_status();
+}
+
+template <int EPI, int WM, int WN, int NT, int WF>
+int launch_shape(TileArgs& a, long blocks, hipStream_t st) {
+  constexpr int TM = Shape<WM, WN, NT, WF>::kTm;
+  a.mtiles = (a.M + TM - 1) / TM;
+  if constexpr (WM == 1) {
+    const long weight_bytes = (EPI == HTN_EPI_SWIGLU ? 2L : 1L) * a.N * a.K * (WF == WF_BF16 ? 2 : 1);
+    if (weight_bytes >= (a.mtiles == 1 ? kStreamOnceBytes : kStreamBytes))
+      return launch_policy<EPI, WM, WN, NT, WF, 2>(a, blocks, st);
+  }
+  return launch_policy<EPI, WM, WN, NT, WF, 0>(a, blocks, st);
 }
 
 template <int EPI, int WF>
