@@ -606,9 +606,13 @@ int choose_splits(int strips, int waves, int K) {
 template <int MT, int S, int EPI, int W, bool NORM>
 int launch_w(RowsArgs& a, hipStream_t st) {
   const int strips = (a.N + kStrip - 1) / kStrip;
-  if (2L * S * a.N * a.K >= (EPI == HTN_EPI_ARGMAX ? kStreamHeadBytes : kStreamBytes))
-    hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, 2>), dim3(strips, a.KS), dim3(W * 64),
-                       0, st, a);
+  // Large weights come here with up to 16 rows (more take the tiles), and
+  // vocabularies with any number.
+  constexpr bool kStreams = MT == 1 || EPI == HTN_EPI_ARGMAX;
+  const bool stream = 2L * S * a.N * a.K >= (EPI == HTN_EPI_ARGMAX ? kStreamHeadBytes : kStreamBytes);
+  if (kStreams && stream)
+    hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, kStreams ? 2 : 0>), dim3(strips, a.KS),
+                       dim3(W * 64), 0, st, a);
   else
     hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, 0>), dim3(strips, a.KS), dim3(W * 64),
                        0, st, a);

@@ -242,18 +242,11 @@ def residual_rows(x, weight, residual):
     return out
 
 
-def splits_k(n, k, rows):
-    """Whether the multi-row projection of a [n, k] weight over `rows` rows
-    (per launch: at most MAX_ROWS) splits K across blocks: its split finish
-    can then also write the next RMSNorm at no extra launch."""
-    rows = max(1, min(rows, MAX_ROWS))
-    return _lib.load().htn_gemm_rows_scratch_bytes(rows, n, k, _lib.EPI_RESIDUAL, 0) > 0
-
-
 def residual_norm_rows(x, weight, residual, gain, eps=1e-6):
     """(out, normed): out = residual_rows(x, weight, residual) and normed its
-    RMSNorm with `gain` (the next layer's input), both written by one launch
-    when the projection splits K."""
+    RMSNorm with `gain` (the next layer's input), written by the finish of a
+    projection that splits K, by the residual add of the library's, else by a
+    launch of its own."""
     _check(x, weight)
     n = weight.shape[0]
     if residual.shape != (x.shape[0], n) or residual.dtype != torch.bfloat16 \

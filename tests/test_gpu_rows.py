@@ -298,8 +298,8 @@ def test_split_down_residual_norm():
                                    (70, 12288, 4096)])
 def test_residual_norm_rows_bit_exact(m, k, n):
     """The fused entry gives the bits of the residual projection followed by
-    the row-wise RMSNorm: the 9728-deep shapes split K and finish both in one
-    launch, the others have no K split and run the two kernels."""
+    the row-wise RMSNorm, on the strips (up to 8 rows, 32 of small weights) and
+    on the tiles, which split K and finish both in one launch."""
     w = nrm(47, (n, k), std=0.02).cuda()
     x, res, g = nrm(48, (m, k)).cuda(), nrm(49, (m, n)).cuda(), nrm(50, (n,)).cuda()
     out, normed = RW.residual_norm_rows(x, w, res, g, 1e-6)
@@ -308,6 +308,28 @@ def test_residual_norm_rows_bit_exact(m, k, n):
     assert torch.equal(normed, rms_norm(ref, g, 1e-6))
     torch.testing.assert_close(out.cpu().float(), Q.output_residual(x.cpu(), w.cpu(), res.cpu()).float(),
                                atol=2e-2, rtol=2e-2)
+
+
+# The strips' own entry (35 rows and more split K and finish both in one launch,
+# 20 keep K whole), whose rows of these sizes the Python operators give the tiles.
+@pytest.mark.parametrize("m,k,n,stride", [(128, 9728, 2560, 9728), (70, 12288, 4096, 12288),
+                                          (35, 9728, 1032, 9736), (20, 9728, 2560, 9728),
+                                          (40, 4096, 1024, 8)])
+def test_strips_residual_norm_entry(m, k, n, stride):
+    from hackthenorth_amd import _lib
+    x = nrm(52, (m * stride + k,)).cuda().as_strided((m, k), (stride, 1))
+    w, res, g = nrm(53, (n, k), std=0.02).cuda(), nrm(54, (m, n)).cuda(), nrm(55, (n,)).cuda()
+    nbytes = _lib.load().htn_gemm_rows_scratch_bytes(m, n, k, _lib.EPI_RESIDUAL_NORM, 0)
+    assert (nbytes > 0) == (m > 32)
+    scratch = torch.full((nbytes // 4 + 4,), float("nan"), device="cuda")
+    out, normed = torch.empty(m, n, dtype=torch.bfloat16, device="cuda"), torch.empty_like(res)
+    _lib.call("htn_gemm_rows_residual_norm", _lib.ptr(x), stride, _lib.ptr(w), n, k, m,
+              _lib.ptr(res), n, _lib.ptr(out), n, _lib.ptr(g), 1e-6, _lib.ptr(normed),
+              _lib.ptr(scratch), _lib.stream(x.device))
+    assert torch.equal(normed, rms_norm(out, g, 1e-6))
+    torch.testing.assert_close(
+        out.cpu().float(), Q.output_residual(x.cpu(), w.cpu(), res.cpu()).float(),
+        atol=2e-2, rtol=2e-2)
 
 
 @pytest.mark.parametrize("length", [2, 5, 8])
