@@ -58,6 +58,7 @@ SIGNATURES = {
     "htn_gemm_tiles_scratch_bytes": [_I64, _I64, _I64, _I],
     "htn_gemm_tiles": [_P, _I64, _P, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _P, _P],
     "htn_gemm_tiles_w8_scratch_bytes": [_I64, _I64, _I64, _I, _I],
+    "htn_gemm_tiles_plan": [_I64, _I64, _I64, _I, _I, _P],
     "htn_gemm_tiles_w8": [_P, _I64, _P, _P, _I, _I64, _I64, _I64, _I, _P, _I64, _P, _I64, _P, _P,
                           _P],
     "htn_gemm_tiles_residual_norm": [_P, _I64, _P, _P, _I, _I64, _I64, _I64, _P, _I64, _P, _I64,

@@ -597,6 +597,11 @@ constexpr TileShape kShapes[] = {
     {2, 4, 5, {{1.11f, 1.11f}, {1.20f, 1.20f}}}, {2, 4, 7, {{1.50f, 1.50f}, {1.52f, 1.52f}}},
     {2, 4, 8, {{1.54f, 1.54f}, {1.68f, 1.68f}}}};
 
+// 8-bit weights are never best on the eight-wave tiles of 128 and 160 rows: two
+// four-wave blocks on a CU do the same rows by 256 weight rows in less (0.97
+// and 1.08 us a step against 1.06 and 1.20).
+constexpr bool built_w8(int wm, int wn, int nt) { return wm * wn < 8 || nt > 5; }
+
 // A launch's time by those coefficients: per XCD, `blocks` blocks of `steps`
 // k steps in rounds of two per CU (one, for eight waves), no less than the
 // weights take from HBM, the launch itself, and for a k split its finish: a
@@ -630,6 +635,7 @@ TilePlan plan_tiles(long rows, long n, long k, int epilogue, int format) {
   float best = 0.f;
   for (const TileShape& sh : kShapes) {
     if (argmax && (sh.wm != 1 || sh.nt > 2)) continue;
+    if (format != 0 && !built_w8(sh.wm, sh.wn, sh.nt)) continue;
     const long tm = 16L * sh.nt * sh.wm, tn = 32L * sh.wm * sh.wn / (sw ? 2 : 1);
     const long ntiles = (n + tn - 1) / tn;
     const long per_xcd = (ntiles + 7) / 8 * ((rows + tm - 1) / tm);
@@ -658,6 +664,13 @@ long tiles_scratch_bytes(const TilePlan& p, long rows) {
   return p.ksplit > 1 ? static_cast<long>(p.ksplit) * rows * p.part_rs * 4 : p.keys_bytes;
 }
 
+// Whether tiles of one wave along the rows load a [n, k] weight (twice n rows
+// for SwiGLU) past the caches.
+bool streamed(long mtiles, long n, long k, int epilogue, int format) {
+  const long bytes = (epilogue == HTN_EPI_SWIGLU ? 2 : 1) * n * k * (format == 0 ? 2 : 1);
+  return bytes >= (mtiles == 1 ? kStreamOnceBytes : kStreamBytes);
+}
+
 template <int EPI, int WM, int WN, int NT, int WF, int AUX>
 int launch_policy(const TileArgs& a, long blocks, hipStream_t st) {
   using S = Shape<WM, WN, NT, WF>;
@@ -676,8 +689,7 @@ int launch_shape(TileArgs& a, long blocks, hipStream_t st) {
   constexpr int TM = Shape<WM, WN, NT, WF>::kTm;
   a.mtiles = (a.M + TM - 1) / TM;
   if constexpr (WM == 1) {
-    const long weight_bytes = (EPI == HTN_EPI_SWIGLU ? 2L : 1L) * a.N * a.K * (WF == WF_BF16 ? 2 : 1);
-    if (weight_bytes >= (a.mtiles == 1 ? kStreamOnceBytes : kStreamBytes))
+    if (streamed(a.mtiles, a.N, a.K, EPI, WF))
       return launch_policy<EPI, WM, WN, NT, WF, 2>(a, blocks, st);
   }
   return launch_policy<EPI, WM, WN, NT, WF, 0>(a, blocks, st);
@@ -697,11 +709,14 @@ int launch_tiles(TileArgs& a, const TilePlan& p, hipStream_t st) {
       case 223: return launch_shape<EPI, 2, 2, 3, WF>(a, p.blocks, st);
       case 224: return launch_shape<EPI, 2, 2, 4, WF>(a, p.blocks, st);
       case 225: return launch_shape<EPI, 2, 2, 5, WF>(a, p.blocks, st);
-      case 244: return launch_shape<EPI, 2, 4, 4, WF>(a, p.blocks, st);
-      case 245: return launch_shape<EPI, 2, 4, 5, WF>(a, p.blocks, st);
       case 247: return launch_shape<EPI, 2, 4, 7, WF>(a, p.blocks, st);
-      default: return launch_shape<EPI, 2, 4, 8, WF>(a, p.blocks, st);
+      case 248: return launch_shape<EPI, 2, 4, 8, WF>(a, p.blocks, st);
+      default: break;
     }
+    if constexpr (WF == WF_BF16)
+      return p.nt == 4 ? launch_shape<EPI, 2, 4, 4, WF>(a, p.blocks, st)
+                       : launch_shape<EPI, 2, 4, 5, WF>(a, p.blocks, st);
+    return HTN_EUNSUPPORTED;  // the plan picks no other shape
   }
 }
 
@@ -816,6 +831,20 @@ extern "C" int64_t htn_gemm_tiles_w8_scratch_bytes(int64_t rows, int64_t n, int6
       !known_epilogue(epilogue, format))
     return 0;
   return tiles_scratch_bytes(plan_tiles(rows, n, k, epilogue, format), rows);
+}
+
+extern "C" int htn_gemm_tiles_plan(int64_t rows, int64_t n, int64_t k, int epilogue,
+                                   int weight_format, int32_t* plan) {
+  if (!plan || rows <= 0 || n <= 0 || k <= 0 || k % kTk || weight_format < 0 ||
+      weight_format > HTN_WEIGHT_FP8_E4M3 || !known_epilogue(epilogue, weight_format))
+    return HTN_EINVAL;
+  const TilePlan p = plan_tiles(rows, n, k, epilogue, weight_format);
+  const long tm = 16L * p.nt * p.wm;
+  plan[0] = static_cast<int32_t>(tm);
+  plan[1] = 32 * p.wm * p.wn;
+  plan[2] = p.ksplit;
+  plan[3] = p.wm == 1 && streamed((rows + tm - 1) / tm, n, k, epilogue, weight_format);
+  return HTN_OK;
 }
 
 extern "C" int htn_gemm_tiles(const void* x, int64_t x_stride, const void* w, int64_t n,

@@ -278,6 +278,13 @@ int htn_gemm_tiles_w8(const void* x, int64_t x_stride, const void* w, const floa
                       const void* residual, int64_t res_stride, void* y, int64_t y_stride,
                       int64_t* tokens, void* scratch, htn_stream_t stream);
 
+/* The launch that htn_gemm_tiles (weight_format 0) and htn_gemm_tiles_w8 choose
+ * for these sizes when given scratch: plan[0] rows by plan[1] weight rows per
+ * block, plan[2] k splits, plan[3] whether the weights are loaded past the
+ * caches. */
+int htn_gemm_tiles_plan(int64_t rows, int64_t n, int64_t k, int epilogue, int weight_format,
+                        int32_t* plan);
+
 /* The residual projection of htn_gemm_tiles (weight_format 0, w_scale unused)
  * or htn_gemm_tiles_w8, and normed[m, :n] = rms_norm(y[m]) with `gain`: in the
  * k split's finish when the tiles split k, else one launch more; the same bits

@@ -25,6 +25,14 @@ CASES = [(2, 40, 64), (16, 136, 192), (17, 1000, 2560), (33, 136, 512), (48, 264
          (160, 264, 9728), (201, 1544, 1024), (225, 5128, 640), (300, 6144, 1024),
          (513, 2560, 2048), (160, 12296, 512), (225, 12296, 640), (300, 12296, 640),
          (450, 8200, 1024), (500, 12288, 512), (700, 6152, 640), (1000, 6152, 640)]
+# With these, every tile that the plan picks for bf16 and for 8-bit weights in
+# each epilogue, with its k split and whole, its weights cached and streamed
+# (tests/test_rows_routes.py looks them up).
+COVER = [(523, 528, 64), (1353, 16, 1792), (2, 13688, 768), (2, 1992, 5312), (18, 5168, 2048),
+         (34, 6848, 2112), (1227, 1032, 3840), (198, 14112, 6976), (1337, 5632, 64),
+         (42, 22944, 704), (293, 1416, 8256), (1839, 1096, 9472), (17, 17000, 640),
+         (653, 13320, 64), (696, 16504, 64), (67, 568, 3584), (397, 320, 6784), (884, 552, 7360),
+         (1375, 4240, 64), (196, 2944, 3328), (17, 12296, 448), (235, 5448, 6784)]
 
 
 def bf16(seed, *shape, std=1.0):
@@ -41,6 +49,26 @@ def weight(fmt, n, k, seed):
     codes = q.data.view(torch.int8 if fmt == "int8" else torch.float8_e4m3fn)
     values = codes.float().double() * q.scale.double()[:, None]
     return QuantizedWeight(q.data.cuda(), q.scale.cuda(), fmt), values
+
+
+def gpu_operands(fmt, m, n, k, seed=20):
+    """x [m, k] and a [2n, k] weight, made on the GPU: (x, weight, its first n
+    rows, float64 values)."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def normal(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    x = normal(m, k)
+    if fmt == "bf16":
+        w = normal(2 * n, k) * 0.02
+        return x, w, w[:n], w.double()
+    scale = torch.empty(2 * n, device="cuda").uniform_(0.8, 1.2, generator=g) * 0.02 / 30
+    codes = normal(2 * n, k).float() * 30
+    codes = codes.round().clamp(-127, 127).to(torch.int8) if fmt == "int8" \
+        else codes.to(torch.float8_e4m3fn)
+    data = codes.view(torch.uint8)
+    return x, QuantizedWeight(data, scale, fmt), QuantizedWeight(data[:n], scale[:n], fmt), \
+        codes.double() * scale.double()[:, None]
 
 
 def check_store(got, x, values):
@@ -70,6 +98,108 @@ def test_tiles_match_the_exact_product(fmt, m, n, k):
     torch.testing.assert_close(RW._tiles(xd, w, n, RW._lib.EPI_SWIGLU).cpu().float(),
                                torch.nn.functional.silu(gu[:, :n]) * gu[:, n:],
                                atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", COVER)
+def test_every_tile_of_the_plan(fmt, m, n, k):
+    x, w, half, values = gpu_operands(fmt, m, n, k)
+    check_store(RW._tiles(x, half, n, RW._lib.EPI_STORE), x, values[:n])
+    y = (x.double() @ values.T).to(torch.bfloat16).float()
+    res, gain = bf16(21, m, n).cuda(), bf16(22, n).cuda()
+    if n > 16384:  # past the row-wise norm's widest rows
+        out = RW._tiles(x, half, n, RW._lib.EPI_RESIDUAL, residual=res)
+    else:
+        out, normed = RW._tiles_residual_norm(x, half, res, gain, 1e-6)
+        if n <= 8192:
+            assert torch.equal(normed, rms_norm(out, gain, 1e-6))
+    torch.testing.assert_close(out.float(), y[:, :n] + res.float(), atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(RW._tiles(x, w, n, RW._lib.EPI_SWIGLU).float(),
+                               torch.nn.functional.silu(y[:, :n]) * y[:, n:],
+                               atol=2e-2, rtol=2e-2)
+
+
+# Rows and widths on tiles of 16, 32, 48, 64, 96, 128, 160, 224 and 256 rows.
+FORM_CASES = [(3, 137, 1088), (20, 1001, 4096), (40, 1003, 4096), (70, 2050, 2560), (97, 522, 2048),
+              (129, 2563, 1088), (201, 1541, 1024), (198, 14113, 512), (653, 13321, 64),
+              (696, 16505, 64), (235, 5449, 6784), (884, 553, 7360)]
+
+
+def tiles_abi(fmt, x, w, n, epilogue, residual=None, y_stride=None, y_offset=0, split=True):
+    """The C entry on rows of any stride; y [m, n] of stride `y_stride` from
+    `y_offset` elements into a NaN buffer, of which nothing else may change."""
+    lib, (m, k) = RW._lib, x.shape
+    data, scale, code = RW._weight(w)
+    nbytes = lib.load().htn_gemm_tiles_w8_scratch_bytes(m, n, k, epilogue, code) if split else 0
+    scratch = torch.full((nbytes // 4 + 4,), float("nan"), device="cuda") if nbytes else None
+    stride = n if y_stride is None else y_stride
+    buffer = torch.full((m * stride + y_offset + 8,), float("nan"), dtype=torch.bfloat16,
+                        device="cuda")
+    y = buffer[y_offset:y_offset + m * stride].view(m, stride)
+    head = (lib.ptr(x), x.stride(0), lib.ptr(data))
+    tail = (n, k, m, epilogue, lib.ptr(residual), residual.stride(0) if residual is not None else 0,
+            lib.ptr(y), stride)
+    if code:
+        lib.call("htn_gemm_tiles_w8", *head, lib.ptr(scale), code, *tail, None, lib.ptr(scratch),
+                 lib.stream(x.device))
+    else:
+        lib.call("htn_gemm_tiles", *head, *tail, lib.ptr(scratch), lib.stream(x.device))
+    assert bool(buffer[:y_offset].isnan().all()) and bool(y[:, n:].isnan().all()) \
+        and bool(buffer[y_offset + m * stride:].isnan().all())
+    return y[:, :n]
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("m,n,k", FORM_CASES)
+def test_tiles_take_any_row_stride_and_odd_widths(fmt, split, m, n, k):
+    """Padded input rows, residual rows and outputs; widths off the four columns
+    of a lane; for 8-bit weights outputs of odd strides at odd addresses; with
+    scratch and without (each tile's k range whole)."""
+    x, w, half, values = gpu_operands(fmt, m, n, k)
+    wide = torch.full((m, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, :k] = x
+    padded = torch.zeros(m, n + 3, dtype=torch.bfloat16, device="cuda")
+    padded[:, :n] = bf16(23, m, n).cuda()
+    res = padded[:, :n]
+    stride, offset = (n + (-n) % 4, 0) if fmt == "bf16" else (n + 2 + n % 2, 1)
+    y = (x.double() @ values.T).to(torch.bfloat16).float()
+    form = dict(y_stride=stride, y_offset=offset, split=split)
+    check_store(tiles_abi(fmt, wide[:, :k], half, n, RW._lib.EPI_STORE, **form), x, values[:n])
+    torch.testing.assert_close(
+        tiles_abi(fmt, wide[:, :k], half, n, RW._lib.EPI_RESIDUAL, res, **form).float(),
+        y[:, :n] + res.float(), atol=2e-2, rtol=2e-2)
+    torch.testing.assert_close(
+        tiles_abi(fmt, wide[:, :k], w, n, RW._lib.EPI_SWIGLU, **form).float(),
+        torch.nn.functional.silu(y[:, :n]) * y[:, n:], atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(5, 264, 2048), (40, 1000, 512), (129, 520, 2048), (201, 14112, 512),
+                                   (300, 12296, 640)])
+def test_tiles_keep_nonfinite_values_to_their_rows_and_columns(fmt, m, n, k):
+    """Rows of x with an infinity or a NaN and weight rows with one (8-bit: an
+    fp8 NaN code, an infinite scale) give what the product gives, and every
+    other output stays finite."""
+    x, _, half, values = gpu_operands(fmt, m, n, k)
+    values = values[:n].clone()
+    x[1, k // 2], x[m - 1, 3] = float("inf"), float("nan")
+    if fmt == "bf16":
+        half[n // 2, 7] = float("-inf")
+        values[n // 2, 7] = float("-inf")
+    elif fmt == "fp8_e4m3":
+        half.data[n // 2, 7] = 0x7F
+        values[n // 2, 7] = float("nan")
+    exact = x.double() @ values.T
+    if fmt == "int8":
+        half.scale[n // 2] = float("inf")
+        exact[:, n // 2] *= float("inf")
+    got = RW._tiles(x, half, n, RW._lib.EPI_STORE).double()
+    assert torch.equal(got.isnan(), exact.isnan()) and torch.equal(got.isposinf(), exact.isposinf())
+    assert torch.equal(got.isneginf(), exact.isneginf())
+    finite = exact.isfinite()
+    assert int((~finite).sum()) <= 2 * n + m
+    torch.testing.assert_close(got[finite], exact[finite], atol=2e-2, rtol=2e-2)
 
 
 @pytest.mark.parametrize("fmt", FORMATS[1:])

@@ -1,11 +1,16 @@
 """Which kernel the multi-row projections take for rows of unusual strides and
 widths: what the strips and the library accept is not sent to the tiles, which
 refuse it. The routes are looked up on the CPU, the results compared on the GPU."""
+import ctypes
+import random
+
 import pytest
 import torch
 
+from hackthenorth_amd import _lib
 from hackthenorth_amd.kernels import rows as RW
 from hackthenorth_amd.kernels.rmsnorm import rms_norm
+from test_gpu_tiles import CASES, COVER
 
 
 def matrix(rows, cols, layout, device="cpu", seed=0):
@@ -53,6 +58,29 @@ def test_residual_norm_of_a_prompt_leaves_what_the_tiles_refuse_to_the_library(r
     for off in (8, 40):  # the library takes every multiple of eight
         assert not RW.norm_tiled(matrix(rows, k + off, "plain"),
                                  torch.empty(n, k + off, dtype=torch.bfloat16), res)
+
+
+def test_tile_cases_cover_the_plan():
+    """Every launch the plan picks over sizes drawn from 2 to 2000 rows, widths
+    from 16 to 23000 and k to 12000 (256 CUs, as on the device): tile, k split or
+    whole, cached or streamed weights, per epilogue, bf16 and 8-bit."""
+    lib, out = _lib.load(), (ctypes.c_int32 * 4)()
+
+    def launches(rows, n, k):
+        found = set()
+        for epilogue in (_lib.EPI_STORE, _lib.EPI_RESIDUAL, _lib.EPI_SWIGLU):
+            for fmt in (0, 1):
+                assert lib.htn_gemm_tiles_plan(rows, n, k, epilogue, fmt, out) == _lib.HTN_OK
+                assert (out[2] > 1) == (lib.htn_gemm_tiles_w8_scratch_bytes(
+                    rows, n, k, epilogue, fmt) > 0)
+                found.add((epilogue, fmt, out[0], out[1], out[2] > 1, out[3]))
+        return found
+    covered = set().union(*(launches(*c) for c in CASES + COVER))
+    rng, drawn = random.Random(1), set()
+    for _ in range(20000):
+        drawn |= launches(int(2 ** rng.uniform(1, 11)), 8 * int(2 ** rng.uniform(1, 11.5)),
+                          64 * int(2 ** rng.uniform(0, 7.6)))
+    assert drawn <= covered, sorted(drawn - covered)
 
 
 @pytest.mark.gpu
