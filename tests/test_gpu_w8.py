@@ -183,3 +183,45 @@ def test_w8_layers_and_teacher_forced_ids_match_oracle(fmt):
         o = int(logits[i].to(torch.bfloat16).float().argmax())
         if p != o:
             assert float(logits[i].max() - logits[i][p]) < 2e-2, (i, p, o)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("width", [2, 5, 16])
+def test_w8_verify_rows_against_steps(fmt, width):
+    """A verify pass's rows (matrix-core tiles) against the same tokens in single
+    steps (GEMVs). They sum each dot product in another order, so a value may
+    round to bf16 the other way at each of a layer's seven boundaries, and at a
+    near-tie a row may pick another token than a step: hidden rows within
+    2^-9 sqrt(7 layers) of each other, K/V rows alike, ids whose logit lies
+    within four such shares of the logits' rms of the step's best."""
+    prompt, tokens = Q.prompt_ids(12, 97, seed=1), Q.prompt_ids(width, 97, seed=2)
+    model, _, shape = _tiny(fmt, len(prompt) + width)
+    bar = 2.0 ** -9 * (7 * shape.layers) ** 0.5
+    start = len(prompt)
+    with torch.inference_mode():
+        first = D.KVCache(model, 1, start + width)
+        rotary = D.RotaryTable(model, first.capacity)
+        D.forward(model, torch.tensor([prompt], device="cuda"), first,
+                  torch.arange(start, device="cuda"), rotary=rotary)
+        other = D.KVCache(model, 1, start + width)
+        other.storage.copy_(first.storage)
+        rows, steps = [], []
+        ids = D.forward(model, torch.tensor([tokens], device="cuda"), first,
+                        start + torch.arange(width, device="cuda"), last_only=False,
+                        rotary=rotary, record=rows)
+        for i, t in enumerate(tokens):
+            record = []
+            D.forward(model, torch.tensor([[t]], device="cuda"), other,
+                      torch.tensor([start + i], device="cuda"), rotary=rotary, record=record)
+            steps.append(record[-1].view(-1))
+        steps = torch.stack(steps)
+
+        def close(a, b):
+            return float((a.double() - b.double()).norm() / b.double().norm()) <= bar
+        assert close(rows[-1][0], steps)
+        assert close(first.storage, other.storage)
+        for i in range(width):
+            logits = P.norm_projection(steps[i:i + 1], model.norm.weight, model.lm_head_weight,
+                                       model.norm.variance_epsilon).float().view(-1)
+            deficit = float(logits.max() - logits[int(ids[0, i])])
+            assert deficit <= 4 * bar * float(logits.square().mean().sqrt()), (i, deficit)
