@@ -13,11 +13,23 @@ from hackthenorth_amd.kernels.attention import grouped_attention
 pytestmark = pytest.mark.gpu
 
 # (batch, heads, kv heads, queries, first position): one and four sequences, a
-# ragged last tile, odd group sizes (one head per block), eight heads on one kv
-# head, and just past one and past two blocks per CU (the order of the query
-# tiles turns between them).
+# ragged last tile, odd group sizes (one head per block, up to and past two
+# blocks per CU), eight heads on one kv head, just past one and past two blocks
+# per CU (the order of the query tiles turns between them), and many sequences of
+# a few queries.
 CASES = [(1, 32, 8, 1089, 0), (1, 32, 8, 2113, 0), (4, 32, 8, 300, 37), (1, 24, 8, 1500, 0),
-         (1, 32, 32, 1100, 5), (2, 16, 8, 1111, 100), (1, 8, 1, 4200, 0), (3, 32, 8, 500, 700)]
+         (1, 24, 8, 2900, 0), (2, 24, 8, 700, 3), (1, 32, 32, 1100, 5), (2, 16, 8, 1111, 100),
+         (1, 8, 1, 4200, 0), (3, 32, 8, 500, 700), (32, 32, 8, 16, 40), (64, 32, 8, 9, 500),
+         (40, 16, 8, 33, 0), (32, 24, 8, 16, 40)]
+
+
+def slices(queries):
+    """Ranges of up to 64 queries, whole 64-query tiles of the call, and the last
+    64 once more where the last tile has too few for the prefill kernels."""
+    ranges = [(s, min(queries, s + 64)) for s in range(0, queries, 64)]
+    if ranges[-1][1] - ranges[-1][0] <= 8:  # a verify pass's rows: another kernel
+        ranges[-1] = (max(0, queries - 64), queries)
+    return ranges
 
 
 @pytest.mark.parametrize("order", ["causal", "shuffled"])
@@ -38,14 +50,10 @@ def test_long_prompt_equals_short_calls(batch, heads, kv_heads, queries, first, 
     whole = torch.empty(batch, queries, heads, 128, dtype=torch.bfloat16,
                         device="cuda").transpose(1, 2)
     grouped_attention(q, k, v, positions, out=whole)
-    step = 64
     for b in range(batch):
-        for s in range(0, queries, step):
-            part = q[b:b + 1, :, s:s + step]
-            if part.shape[2] <= 8:  # a verify pass's rows: another kernel
-                continue
-            short = grouped_attention(part, k[b:b + 1], v[b:b + 1], positions[s:s + step])
-            assert torch.equal(whole[b:b + 1, :, s:s + step], short)
+        for s, e in slices(queries):
+            short = grouped_attention(q[b:b + 1, :, s:e], k[b:b + 1], v[b:b + 1], positions[s:e])
+            assert torch.equal(whole[b:b + 1, :, s:e], short)
 
 
 # (batch, heads, kv heads, queries, first position): first positions at which a
