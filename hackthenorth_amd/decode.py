@@ -26,7 +26,7 @@ from .kernels.fused import norm_rope_cache
 from .kernels.greedy import greedy_head
 from .kernels.projection import norm_projection, output_projection_residual
 from .kernels.rows import (greedy_rows, projection_rows, residual_norm_rows, residual_rows,
-                           streams_head, swiglu_rows, tiled)
+                           streams_head, swiglu_rows, writes_norm)
 from .speculate import draft_width, verified_tokens
 
 
@@ -211,7 +211,7 @@ def _forward_rows(model, token_ids, cache, positions, last_only, position_embedd
             # The tiles write the next RMSNorm with their residual projections (in
             # the split finish, where k splits), the library's row-wise residual
             # add too; after strips the next projection normalises its rows itself.
-            if tiled(a, layer.o_weight):
+            if writes_norm(a, layer.o_weight, h):
                 r, rn = residual_norm_rows(a, layer.o_weight, h, ln2.weight,
                                            ln2.variance_epsilon)
                 m = swiglu_rows(rn, layer.gate_up_weight)
@@ -220,7 +220,7 @@ def _forward_rows(model, token_ids, cache, positions, last_only, position_embedd
                 m = swiglu_rows(r, layer.gate_up_weight, ln2.weight, ln2.variance_epsilon)
             nxt = model.layers[i + 1].input_layernorm if i + 1 < len(model.layers) \
                 else model.norm
-            if tiled(m, layer.down_weight):
+            if writes_norm(m, layer.down_weight, r):
                 h, hn = residual_norm_rows(m, layer.down_weight, r, nxt.weight,
                                            nxt.variance_epsilon)
             else:

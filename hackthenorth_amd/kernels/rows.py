@@ -3,7 +3,7 @@
 The speculative verify pass scores k + 1 tokens in one forward; the reference
 runs its multi-row projections as Triton GEMM tiles (dryft/engine/
 projections.py:168-183, kernels/gateup.py:40-58, kernels/split_down.py:85-101).
-Here few rows (STRIP_ROWS) are one htn_gemm_rows launch (16-column strips, the
+Here few rows (strip_rows) are one htn_gemm_rows launch (16-column strips, the
 RMSNorm inside, plus a K-split reduction when the strips alone cannot fill the
 GPU) and more rows one htn_gemm_tiles launch (LDS-staged output tiles, plus the
 finish of its k split), with the batch-one GEMVs' bf16 rounding boundaries.
@@ -20,19 +20,6 @@ from ..quant import QuantizedWeight
 from .greedy import greedy_head
 
 MAX_ROWS = 128    # rows per htn_gemm_rows launch
-# Rows up to which bf16 projections take the strips: of weights of at least
-# LARGE elements, of those whose shorter side is at least WIDE too, and of
-# smaller ones. Strips / tiles, in us, with the RMSNorm in the strips' QKV and
-# gate/up and in the tiles' O and down:
-#   8B, QKV, O, gate/up, down: 9 rows 16, 9, 34, 20 / 14, 14, 32, 29; 16 rows 20,
-#   10, 38, 24 / 15, 14, 32, 31 (a slice of the model: 432 / 482 and 486 / 496);
-#   17 rows, two row tiles per strip, 23, 11, 41, 26 / 15, 14, 33, 30;
-#   4B: 9 rows 12, 8, 24, 14 / 11, 11, 21, 16; 16 rows 15, 9, 28, 18 / 12, 11,
-#   21, 17 (O and down are 160 strips of 16 columns, too few for the CUs; from
-#   4096 columns on there is a strip per CU);
-#   0.6B: 8 rows 5, 5, 6, 5 / 8, 10, 8, 11; 32 rows 9, 7, 10, 9 / 8, 10, 8, 11.
-STRIP_ROWS, WIDE_STRIP_ROWS, SMALL_STRIP_ROWS = 8, 16, 32
-LARGE, WIDE = 8 << 20, 4096
 # Bytes from which a bf16 vocabulary is streamed past the caches, one row of it
 # as the batch-one head (a smaller one is still cached from the last pass: a
 # row without the norm 8.7 us on the strips, 10.6 on the head; 33 MB from HBM
@@ -40,12 +27,16 @@ LARGE, WIDE = 8 << 20, 4096
 STREAM_HEAD_BYTES = 64 << 20
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
-# Rows from which a plain store (QKV) and a residual projection leave the
-# tiles, whose finish writes the next norm too, for the library: 8B at 300
-# rows QKV 32 us on the tiles and 30 through the library, O with its norm 29
+# A plain store (QKV) of LIBRARY_ROWS rows goes to the library, a residual
+# projection with the next norm past them, or past SHALLOW_ROWS where k is
+# under DEEP; a residual projection alone stays on the tiles at any count. 8B at
+# 300 rows QKV 32 us on the tiles and 30 through the library, O with its norm 29
 # and 35, down 59 and 78; at 512 rows 44 / 38, 35 / 39, 79 / 90; at 2048 the
-# library wins throughout (QKV 85 us against 137).
-LIBRARY_ROWS = 512
+# library wins throughout (QKV 85 us against 137). Shorter k leave the tiles'
+# finish a larger share: [2560, 2560] 300 rows 21.7 / 22.3, 512 27.3 / 24.6;
+# [4096, 2048] 24.5 / 24.6 and 30.1 / 27.0; [3072, 3072] 23.3 / 24.1, 450 28.3
+# either way.
+LIBRARY_ROWS, SHALLOW_ROWS, DEEP = 512, 320, 3072
 # Plain products of TILE_ROWS rows or more through hipBLASLt (False: this
 # library's tiled kernel for every prompt projection, e.g. to measure it).
 LIBRARY = True
@@ -153,31 +144,74 @@ def _tiles_residual_norm(x, weight, residual, gain, eps):
     return out, normed
 
 
-def tiled(x, weight):
-    """Whether a projection of these rows takes the tiles: 8-bit weights
-    always, bf16 ones past the strips' rows whose output rows the tiles' 8-byte
-    stores and whose input strides their 32-bit offsets cover, unless the input
-    rows overlap (an expanded row, sliding windows: the strips read those);
-    TILE_ROWS rows or more have no other kernel."""
-    if isinstance(weight, QuantizedWeight):
+def strip_rows(n, k, swiglu=False, norm=False):
+    """Rows up to which a bf16 [n, k] projection takes the strips (swiglu: n
+    counts the gate and up rows; norm: with the input rows' RMSNorm).
+
+    A strip re-reads its rows' x per 16 columns, so its time grows with rows and
+    k (17, 33 and 65 rows begin another row tile), while the tiles pay a second
+    launch for their k split and one for a norm first. Strips / tiles in us,
+    weights from HBM:
+    [4096, 1024] 64 rows 7.3 / 8.1; [2048, 2048] 32 rows 7.6 / 9.0, 48 9.8 / 9.1;
+    [4096, 2048] 32 rows 8.0 / 9.3; [6144, 2560] 16 rows 11.7 / 11.8, 24 13.8 /
+    12.2; [24576, 4096] 16 rows 32.8 / 32.5, 17 39.0 / 33.0. SwiGLU of few
+    columns: [6144, 2048] 24 rows 12.0 / 14.8. Past k = 4096 they cross by 12
+    rows ([2560, 9728] 8 rows 13.7 / 15.2, 12 15.8 / 15.3; [5120, 5120] 8 rows 15
+    / 14), but not where whole rounds of strips fill the CUs ([4096, 12288] 16
+    rows 23.8 / 28.1) nor with a norm in the strips' launch ([2048, 6144] 16
+    rows 16.8 / 18.6)."""
+    if k <= 1024 and n * k <= 5 << 20:
+        return 64
+    if k <= 3072 and n * k < 12 << 20 or swiglu and n <= 8192 and k <= 5120:
+        return 32
+    if k <= 4096 or n % 4096 == 0 or norm and n * k < 20 << 20:
+        return 16
+    return 12 if k <= 8192 else 8
+
+
+def norm_strip_rows(n, k):
+    """strip_rows of a residual projection whose rows the next projection
+    normalises: on the strips in that one's launch, at its expense, on the tiles
+    in this one's finish. Both together, strips / tiles, 12 rows: 4B O and gate/up
+    33.5 / 31.9, down and QKV 29.3 / 27.0, 8 rows 31.2 / 31.3 and 25.6 / 25.2; 8B
+    44.3 / 45.5 and 39.8 / 43.5, 16 rows 47.1 / 46.7 and 44.3 / 44.1; a 2048-wide
+    model's down and QKV 19.1 / 19.6."""
+    return 8 if n * k >= 10 << 20 and n > 2048 and n % 4096 else strip_rows(n, k)
+
+
+def _tileable(x, weight):
+    """Rows and output widths that the tiles' 8-byte stores and 32-bit offsets
+    cover; not rows that overlap (an expanded row, sliding windows), which the
+    strips read."""
+    return weight.shape[0] % 8 == 0 and x.shape[1] <= x.stride(0) < 1 << 22
+
+
+def tiled(x, weight, swiglu=False, norm=False):
+    """Whether a projection of these rows (strip_rows) takes the tiles: 8-bit weights always,
+    bf16 ones past the strips' rows; TILE_ROWS rows or more have no other kernel."""
+    if isinstance(weight, QuantizedWeight) or x.shape[0] >= TILE_ROWS:
         return True
-    rows = x.shape[0]
-    strips = SMALL_STRIP_ROWS if weight.numel() < LARGE \
-        else WIDE_STRIP_ROWS if min(weight.shape) >= WIDE else STRIP_ROWS
-    return rows >= TILE_ROWS or (rows > strips and weight.shape[0] % 8 == 0
-                                 and x.shape[1] <= x.stride(0) < 1 << 22)
+    return x.shape[0] > strip_rows(*weight.shape, swiglu, norm) and _tileable(x, weight)
 
 
 def norm_tiled(x, weight, residual):
     """Whether a residual projection with the next RMSNorm takes the tiles: of
-    a prompt's rows up to LIBRARY_ROWS, and there not those of which the
-    library's product and the row-wise residual add take more: widths off the
+    a prompt's rows up to LIBRARY_ROWS (SHALLOW_ROWS where k < DEEP), and there
+    not those of which the library's product and the row-wise residual add take more: widths off the
     64-wide k steps, residual rows that overlap, far strides."""
-    if not prompt(x, weight):
-        return tiled(x, weight)
+    if isinstance(weight, QuantizedWeight):
+        return True
     n, k = weight.shape
-    return x.shape[0] <= LIBRARY_ROWS and k % 64 == 0 and residual.stride(0) >= n \
-        and x.stride(0) < 1 << 22
+    if not prompt(x, weight):
+        return x.shape[0] > norm_strip_rows(n, k) and _tileable(x, weight)
+    return x.shape[0] <= (LIBRARY_ROWS if k >= DEEP else SHALLOW_ROWS) and k % 64 == 0 \
+        and residual.stride(0) >= n and x.stride(0) < 1 << 22
+
+
+def writes_norm(x, weight, residual):
+    """Whether a layer's residual projection is to write the next RMSNorm too
+    (residual_norm_rows): on the tiles and after the library's product."""
+    return prompt(x, weight) or norm_tiled(x, weight, residual)
 
 
 def _scratch(device, rows, n, k, epilogue, norm):
@@ -217,7 +251,7 @@ def projection_rows(x, weight, gain=None, eps=1e-6):
     """bf16(W x_m) for every row m of x [M, K]; gain applies RMSNorm first."""
     _check(x, weight)
     _lib.require_gpu(x, _weight(weight)[0], gain)
-    if tiled(x, weight):
+    if tiled(x, weight, norm=gain is not None):
         run = _prefill if prompt(x, weight) else _tiles
         return run(x, weight, weight.shape[0], _lib.EPI_STORE, gain=gain, eps=eps)
     out = torch.empty((x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device)
@@ -294,7 +328,7 @@ def swiglu_rows(x, gate_up_weight, gain=None, eps=1e-6):
         raise ValueError("packed gate/up width must be even")
     _lib.require_gpu(x, _weight(gate_up_weight)[0], gain)
     n = gate_up_weight.shape[0] // 2
-    if tiled(x, gate_up_weight):
+    if tiled(x, gate_up_weight, True, gain is not None):
         run = _prefill if prompt(x, gate_up_weight) else _tiles
         return run(x, gate_up_weight, n, _lib.EPI_SWIGLU, gain=gain, eps=eps)
     out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)

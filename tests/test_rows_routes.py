@@ -29,17 +29,40 @@ def matrix(rows, cols, layout, device="cpu", seed=0):
     return normal(rows, cols)
 
 
-@pytest.mark.parametrize("n,k,strips", [(1024, 2048, 32), (2560, 9728, 8), (6144, 2560, 8),
-                                        (4096, 12288, 16), (24576, 4096, 16)])
-def test_strips_end_by_weight_size(n, k, strips):
-    """The last row count on the strips: small weights, large ones, and large ones
-    with at least a strip of 16 columns per CU in every projection of the model."""
+# The projections of models 1024, 2048, 2560, 4096 and 5120 wide: the last row
+# count on the strips, without and with an input norm, and for residual
+# projections with the next norm.
+@pytest.mark.parametrize("n,k,swiglu,plain,with_input_norm,with_next_norm", [
+    (4096, 1024, False, 64, 64, None), (1024, 2048, False, 32, 32, 32),
+    (6144, 1024, True, 32, 32, None), (1024, 3072, False, 32, 32, 32),
+    (4096, 2048, False, 32, 32, None), (2048, 2048, False, 32, 32, 32),
+    (12288, 2048, True, 16, 16, None), (2048, 6144, False, 12, 16, 12),
+    (6144, 2560, False, 16, 16, None), (2560, 4096, False, 16, 16, 8),
+    (19456, 2560, True, 16, 16, None), (2560, 9728, False, 8, 8, 8),
+    (6144, 4096, False, 16, 16, None), (4096, 4096, False, 16, 16, 16),
+    (24576, 4096, True, 16, 16, None), (4096, 12288, False, 16, 16, 16),
+    (7168, 5120, False, 12, 12, None), (5120, 5120, False, 12, 12, 8),
+    (5120, 17408, False, 8, 8, 8), (6144, 2048, True, 32, 32, None)])
+def test_strips_end_by_weight_size(n, k, swiglu, plain, with_input_norm, with_next_norm):
     w = torch.empty(n, k, dtype=torch.bfloat16, device="meta")
-    for rows in (strips, strips + 1):
-        assert RW.tiled(torch.empty(rows, k, device="meta"), w) == (rows > strips)
+    for last, norm in ((plain, False), (with_input_norm, True)):
+        for rows in (last, last + 1):
+            x = torch.empty(rows, k, device="meta")
+            assert RW.tiled(x, w, swiglu, norm) == (rows > last)
+    for rows in (with_next_norm, with_next_norm + 1) if with_next_norm else ():
+        x, res = torch.empty(rows, k, device="meta"), torch.empty(rows, n, device="meta")
+        assert RW.norm_tiled(x, w, res) == RW.writes_norm(x, w, res) == (rows > with_next_norm)
 
 
-@pytest.mark.parametrize("rows,n,k", [(17, 4096, 4096), (33, 512, 1024), (100, 512, 1024),
+@pytest.mark.parametrize("n,k,last", [(4096, 4096, 512), (1024, 3072, 512), (1024, 2048, 320)])
+def test_residual_norm_goes_to_the_library_by_rows_and_depth(n, k, last):
+    w = torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+    for rows in (256, last, last + 1):
+        x, res = torch.empty(rows, k, device="meta"), torch.empty(rows, n, device="meta")
+        assert RW.norm_tiled(x, w, res) == (rows <= last) and RW.writes_norm(x, w, res)
+
+
+@pytest.mark.parametrize("rows,n,k", [(17, 4096, 4096), (65, 512, 1024), (100, 512, 1024),
                                       (255, 4096, 4096)])
 def test_overlapping_rows_stay_on_the_strips(rows, n, k):
     w = torch.empty(n, k, dtype=torch.bfloat16)
@@ -48,7 +71,7 @@ def test_overlapping_rows_stay_on_the_strips(rows, n, k):
     assert RW.tiled(matrix(rows, k, "padded"), w) == RW.tiled(matrix(rows, k, "plain"), w)
 
 
-@pytest.mark.parametrize("rows", [256, 300, 512])
+@pytest.mark.parametrize("rows", [256, 300, 320])
 def test_residual_norm_of_a_prompt_leaves_what_the_tiles_refuse_to_the_library(rows):
     n, k = 512, 1024
     w, res = torch.empty(n, k, dtype=torch.bfloat16), matrix(rows, n, "plain")
