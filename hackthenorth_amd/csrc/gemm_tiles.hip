@@ -2,18 +2,19 @@
 // y = x W^T over M rows as a tiled GEMM on the matrix cores, for bf16 weights
 // and for 8-bit ones (int8 or fp8-e4m3fn codes with an fp32 scale per row).
 //
-//  * block = four waves on an output tile of TM rows x 128 weight rows. The
-//    waves stand 2 x 2 (TM = 32 NT: each wave 16 NT rows x 64 weight rows) or,
-//    for at most 48 rows, 1 x 4 (TM = 16 NT: all rows x 32 weight rows);
+//  * block = four waves on an output tile of TM rows x 128 weight rows, or
+//    eight on TM rows x 256. The waves stand 2 x 2 or 2 x 4 (TM = 32 NT: each
+//    wave 16 NT rows x 64 weight rows) or, for tiles of at most 48 rows, 1 x 4
+//    (TM = 16 NT: all rows x 32 weight rows);
 //  * each 64-deep k step stages the x tile (TM rows x 128 bytes) and the
-//    weight tile (128 rows of 128 bytes, or 64 for 8-bit codes) into LDS with
-//    LDS-direct loads, a ring of kStages steps deep: as many as leave room for
-//    two blocks per CU, because what bounds a few hundred rows is the weight
-//    stream, i.e. the bytes in flight, and what bounds more is the matrix
-//    cores, which need a second block's waves while one waits at its barrier.
-//    A wave waits only for the step it is about to multiply (vmcnt counts the
-//    later steps' loads, the same number in every step: steps past the end
-//    are loaded through an empty descriptor, as zeros);
+//    weight tile (128 or 256 rows of 128 bytes, or 64 for 8-bit codes) into LDS
+//    with LDS-direct loads, a ring of kStages steps deep: as many as leave room
+//    for two four-wave blocks per CU or one of eight waves, because what bounds
+//    a few hundred rows is the weight stream, i.e. the bytes in flight, and what
+//    bounds more is the matrix cores, which need other waves while some wait at
+//    a barrier. A wave waits only for the step it is about to multiply (vmcnt
+//    counts the later steps' loads, the same number in every step: steps past
+//    the end are loaded through an empty descriptor, as zeros);
 //  * x chunk c (16 bytes) of row r sits at column c ^ (r & 7), weight chunk c
 //    of an 8-bit row at c ^ ((r >> 2) & 3), so the fragment reads of eight
 //    consecutive lanes hit eight different column groups;
@@ -24,8 +25,9 @@
 //    16 q .. 16 q + 15 and x is read in the same permuted order, which leaves
 //    each dot product unchanged. The row scale multiplies the fp32 sum, as in
 //    the batch-one GEMVs;
-//  * SwiGLU tiles interleave gate and up rows in groups of 16 (32 with 2 x 2
-//    waves), so a lane holds the gate and up dot products of the same outputs;
+//  * SwiGLU tiles interleave gate and up rows in groups of 16 (32 with two
+//    waves along the rows), so a lane holds the gate and up dot products of the
+//    same outputs;
 //  * when the tiles leave block slots empty, each tile's k range splits over
 //    up to 12 blocks; they store fp32 partial sums and a second launch adds
 //    them in split order and applies the epilogue (with the next RMSNorm, when
@@ -41,10 +43,13 @@
 // gate/up 190 -> 67 (605 TFLOP/s, 3.0 TB/s), down 170 -> 51; 0.6B at 100 rows
 // 10 / 13 / 12 / 14 -> 8 / 10 / 8 / 11. 4B at 300 rows, fp8, against the GEMV
 // row by row: 8.4 ms -> 23 + 25 + 42 + 39 us (gate/up 712 TFLOP/s). What bounds
-// them: a CU takes 50 GB/s from HBM and 85-110 from L2 into LDS, whatever the
-// ring's depth, so a tile's staged bytes, (TM + 128) x 128 per step, set the
-// time of a step (18 KB for 16 rows: 0.36 us; 36 KB for 160: 0.9), which is
-// why few rows want narrow tiles on every CU and many want wide ones.
+// them: a CU stages some 50 bytes per ns, x and weights together, whatever the
+// ring's depth (a step of 18 KB for 16 rows takes 0.36 us, of 36 KB for 160
+// rows 0.9). All 256 CUs at that rate would take 12.8 TB/s, twice what the
+// weights come from HBM at: a launch of few rows on every CU is bound by that
+// stream, one that leaves CUs without a block, or whose rows make the x tile
+// most of what is staged, by its CUs. Hence narrow tiles on every CU for few
+// rows and wide ones for many.
 #include "common.h"
 
 namespace htn {
@@ -96,8 +101,8 @@ constexpr long kStreamBytes = 16L << 20, kStreamOnceBytes = 10L << 20;
 constexpr int kMinSplitSteps = 8;     // k steps each split keeps at least
 constexpr int kMaxSplit = 12;
 
-// A tile's shape: waves along the rows (2: 2 x 2 waves; 1: 1 x 4), 16-row x
-// tiles per wave, weight format.
+// A tile's shape: waves along the rows (WM) and the weight rows (WN), 16-row x
+// tiles per wave (NT), weight format.
 template <int WM, int WN, int NT, int WF>
 struct Shape {
   static constexpr int kTm = 16 * NT * WM;
@@ -271,9 +276,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_tiles_kernel(TileArgs a)
   const int nt = g * 8 + (L & 7), mt = q - s * a.mtiles;
   if (nt >= a.ntiles) return;
   const int m0 = mt * TM;
-  // Weight rows of the tile: rows n0 .. n0 + 127, or for SwiGLU 64 output
-  // columns n0 .. n0 + 63 as eight 16-row groups: gate, gate, up, up, twice
-  // (2 x 2 waves), or gate, up, four times.
+  // Weight rows of the tile: kTn rows from n0, or for SwiGLU kTn / 2 output
+  // columns from n0 as 16-row groups: gate, gate, up, up, ... with two waves
+  // along the rows, else gate, up, ....
   const int n0 = nt * (SW ? S::kTn / 2 : S::kTn);
 
   // Staging: a lane of load li takes x row 8 li + lane / 8 and writes position

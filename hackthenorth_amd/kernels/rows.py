@@ -7,11 +7,12 @@ Here few rows (strip_rows) are one htn_gemm_rows launch (16-column strips, the
 RMSNorm inside, plus a K-split reduction when the strips alone cannot fill the
 GPU) and more rows one htn_gemm_tiles launch (LDS-staged output tiles, plus the
 finish of its k split), with the batch-one GEMVs' bf16 rounding boundaries.
-From TILE_ROWS rows on (a prompt's prefill) the plain product of the gate/up
-projection, and from LIBRARY_ROWS on of every projection, runs through
-hipBLASLt (htn_gemm_library) with the epilogues as row-wise launches, where the
-library has an algorithm. 8-bit weights (QuantizedWeight) take
-htn_gemm_tiles_w8 at every row count.
+In a prompt's prefill the plain product of the gate/up projection from
+TILE_ROWS rows on, of a plain store from LIBRARY_ROWS rows on and of a residual
+projection with the next norm past them runs through hipBLASLt
+(htn_gemm_library) with the epilogues as row-wise launches, where the library
+has an algorithm. 8-bit weights (QuantizedWeight) take htn_gemm_tiles_w8 at
+every row count.
 """
 import torch
 
@@ -28,15 +29,15 @@ STREAM_HEAD_BYTES = 64 << 20
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
 # A plain store (QKV) of LIBRARY_ROWS rows goes to the library, a residual
-# projection with the next norm past them, or past SHALLOW_ROWS where k is
-# under DEEP; a residual projection alone stays on the tiles at any count. 8B at
+# projection with the next norm past them, or past WIDE_ROWS where it is wider
+# than deep; a residual projection alone stays on the tiles at any count. 8B at
 # 300 rows QKV 32 us on the tiles and 30 through the library, O with its norm 29
 # and 35, down 59 and 78; at 512 rows 44 / 38, 35 / 39, 79 / 90; at 2048 the
-# library wins throughout (QKV 85 us against 137). Shorter k leave the tiles'
-# finish a larger share: [2560, 2560] 300 rows 21.7 / 22.3, 512 27.3 / 24.6;
-# [4096, 2048] 24.5 / 24.6 and 30.1 / 27.0; [3072, 3072] 23.3 / 24.1, 450 28.3
-# either way.
-LIBRARY_ROWS, SHALLOW_ROWS, DEEP = 512, 320, 3072
+# library wins throughout (QKV 85 us against 137). A short k leaves the tiles'
+# finish a larger share: [5120, 1024] 300 rows 23.4 / 23.2, 512 33.1 / 26.6;
+# [4096, 2048] 24.5 / 24.6 and 30.1 / 27.0; but the 0.6B with its O ([1024,
+# 2048]) on the tiles 259 us of 512 rows for three layers, through the library 264.
+LIBRARY_ROWS, WIDE_ROWS = 512, 320
 # Plain products of TILE_ROWS rows or more through hipBLASLt (False: this
 # library's tiled kernel for every prompt projection, e.g. to measure it).
 LIBRARY = True
@@ -196,15 +197,15 @@ def tiled(x, weight, swiglu=False, norm=False):
 
 def norm_tiled(x, weight, residual):
     """Whether a residual projection with the next RMSNorm takes the tiles: of
-    a prompt's rows up to LIBRARY_ROWS (SHALLOW_ROWS where k < DEEP), and there
-    not those of which the library's product and the row-wise residual add take more: widths off the
+    a prompt's rows up to LIBRARY_ROWS (WIDE_ROWS where n > k), and there not
+    those of which the library's product and the row-wise residual add take more: widths off the
     64-wide k steps, residual rows that overlap, far strides."""
     if isinstance(weight, QuantizedWeight):
         return True
     n, k = weight.shape
     if not prompt(x, weight):
         return x.shape[0] > norm_strip_rows(n, k) and _tileable(x, weight)
-    return x.shape[0] <= (LIBRARY_ROWS if k >= DEEP else SHALLOW_ROWS) and k % 64 == 0 \
+    return x.shape[0] <= (LIBRARY_ROWS if k >= n else WIDE_ROWS) and k % 64 == 0 \
         and residual.stride(0) >= n and x.stride(0) < 1 << 22
 
 
