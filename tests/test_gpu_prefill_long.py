@@ -91,3 +91,25 @@ def test_later_nonfinite_values_reach_no_further_than_in_short_calls(batch, head
             torch.testing.assert_close(whole[:1, :, s:s + 64], short, rtol=0, atol=0,
                                        equal_nan=True)
     assert bool(whole.isfinite().any())
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(32, 8), (24, 8)])
+def test_positions_outside_the_cache_as_in_short_calls(heads, kv_heads):
+    """Queries before the first slot (they see nothing: 0 / 0) and past the last
+    (they see every slot), scattered and as a whole leading tile."""
+    batch, queries, capacity = 4, 512, 300
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+    q = normal(batch, queries, heads, 128).transpose(1, 2)
+    k, v = normal(batch, kv_heads, capacity, 128), normal(batch, kv_heads, capacity, 128)
+    positions = torch.arange(queries, device="cuda") - 90
+    positions[::17] = -3
+    positions[5::23] = capacity + 40
+    whole = grouped_attention(q, k, v, positions)
+    for s in range(0, queries, 64):
+        short = grouped_attention(q[:1, :, s:s + 64], k[:1], v[:1], positions[s:s + 64])
+        torch.testing.assert_close(whole[:1, :, s:s + 64], short, rtol=0, atol=0, equal_nan=True)
+    seen = positions >= 0
+    assert bool(whole[:, :, seen].isfinite().all()) and bool(whole[:, :, ~seen].isnan().all())
