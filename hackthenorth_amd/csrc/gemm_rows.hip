@@ -49,9 +49,11 @@ constexpr int kMaxWaves = 16;
 // The 0.6B's smaller ones, where they stay cached from one pass to the next,
 // lose (O 4.3 -> 4.8, down 4.9 -> 5.7).
 constexpr long kStreamBytes = 16L << 20;
-// A vocabulary smaller than this belongs to a model that the last-level cache
-// holds between passes (33 MB of one, among 125 MB of weights: 8.1 us cached,
-// 9.0 streamed; alone at 86 MB 20.2 / 21.9, but from HBM 23.7 / 23.0).
+// Under 16 rows, a vocabulary smaller than this keeps cached loads: it belongs
+// to a model that the last-level cache holds between passes (33 MB of one, among
+// 125 MB of weights: 2 rows 8.1 us cached, 9.0 streamed; alone at 86 MB 20.2 /
+// 21.9, but from HBM 23.7 / 23.0). With more rows their reads leave the cached
+// stream nothing to gain (a pass of 20 rows 157 us, streamed 153).
 constexpr long kStreamHeadBytes = 64L << 20;
 constexpr int kMaxK = 16384;
 
@@ -609,7 +611,8 @@ int launch_w(RowsArgs& a, hipStream_t st) {
   // Large weights come here with up to 16 rows (more take the tiles), and
   // vocabularies with any number.
   constexpr bool kStreams = MT == 1 || EPI == HTN_EPI_ARGMAX;
-  const bool stream = 2L * S * a.N * a.K >= (EPI == HTN_EPI_ARGMAX ? kStreamHeadBytes : kStreamBytes);
+  const bool small_head = EPI == HTN_EPI_ARGMAX && a.M < 16;
+  const bool stream = 2L * S * a.N * a.K >= (small_head ? kStreamHeadBytes : kStreamBytes);
   if (kStreams && stream)
     hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, kStreams ? 2 : 0>), dim3(strips, a.KS),
                        dim3(W * 64), 0, st, a);

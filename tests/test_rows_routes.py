@@ -155,7 +155,7 @@ def test_small_vocabularies_keep_cached_loads():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("vocab", [32767, 32768])  # either side of the streamed size
-@pytest.mark.parametrize("rows", [1, 3, 17, 40])
+@pytest.mark.parametrize("rows", [1, 3, 15, 16, 17, 40])
 def test_greedy_rows_around_the_streamed_size(vocab, rows):
     x, w = matrix(rows, 1024, "plain", "cuda"), matrix(vocab, 1024, "plain", "cuda", 1)
     gain = matrix(1, 1024, "plain", "cuda", 2)[0]
