@@ -47,14 +47,10 @@ constexpr int kMaxWaves = 16;
 // HBM, 8B: O 9.4 -> 8.4 us, gate/up 39.6 -> 35.4, down 22.3 -> 19.8, head 227
 // -> 200 (6.2 TB/s); 4B: 7.9 -> 7.4, 25.0 -> 23.8, 14.7 -> 14.2, 144 -> 130.
 // The 0.6B's smaller ones, where they stay cached from one pass to the next,
-// lose (O 4.3 -> 4.8, down 4.9 -> 5.7).
+// lose (O 4.3 -> 4.8, down 4.9 -> 5.7), its vocabulary of 33 MB gains: a pass of
+// 2 / 8 rows over three models' 125 MB in turn 122 / 142 us cached, 120 / 138
+// streamed (one model's alone, all of it cached: 108.9 / 129.1 and 109.6 / 129.9).
 constexpr long kStreamBytes = 16L << 20;
-// Under 16 rows, a vocabulary smaller than this keeps cached loads: it belongs
-// to a model that the last-level cache holds between passes (33 MB of one, among
-// 125 MB of weights: 2 rows 8.1 us cached, 9.0 streamed; alone at 86 MB 20.2 /
-// 21.9, but from HBM 23.7 / 23.0). With more rows their reads leave the cached
-// stream nothing to gain (a pass of 20 rows 157 us, streamed 153).
-constexpr long kStreamHeadBytes = 64L << 20;
 constexpr int kMaxK = 16384;
 
 struct RowsArgs {
@@ -114,8 +110,7 @@ constexpr int kPitch = 144;  // bytes per staged 64-element weight row (+16: con
 // across the first weight issue (82-92 VGPRs unbounded: 5 waves per SIMD);
 // bounded to 8 (S = 1, 60 VGPRs) and 6 (S = 2, 80) waves per SIMD without
 // spills (8B 16-row batched step 3634 -> 3657 tok/s, 5-row verify unchanged).
-// AUX: the weight loads' cache policy, 2 (non-temporal) from kStreamBytes
-// (kStreamHeadBytes) on.
+// AUX: the weight loads' cache policy, 2 (non-temporal) from kStreamBytes on.
 template <int MT, int S, int EPI, int W, bool NORM, int AUX>
 __global__ __launch_bounds__(W * 64, NORM && MT == 1 ? (S == 1 ? 8 : 6) : 1) void gemm_rows_kernel(RowsArgs a) {
   preload_rows(a);
@@ -611,9 +606,7 @@ int launch_w(RowsArgs& a, hipStream_t st) {
   // Large weights come here with up to 16 rows (more take the tiles), and
   // vocabularies with any number.
   constexpr bool kStreams = MT == 1 || EPI == HTN_EPI_ARGMAX;
-  const bool small_head = EPI == HTN_EPI_ARGMAX && a.M < 16;
-  const bool stream = 2L * S * a.N * a.K >= (small_head ? kStreamHeadBytes : kStreamBytes);
-  if (kStreams && stream)
+  if (kStreams && 2L * S * a.N * a.K >= kStreamBytes)
     hipLaunchKernelGGL((gemm_rows_kernel<MT, S, EPI, W, NORM, kStreams ? 2 : 0>), dim3(strips, a.KS),
                        dim3(W * 64), 0, st, a);
   else

@@ -22,10 +22,10 @@ from .greedy import greedy_head
 
 MAX_ROWS = 128    # rows per htn_gemm_rows launch
 # Bytes from which a bf16 vocabulary is streamed past the caches, one row of it
-# as the batch-one head (a smaller one is still cached from the last pass: a
-# row without the norm 8.7 us on the strips, 10.6 on the head; 33 MB from HBM
-# 12.1 / 10.2).
-STREAM_HEAD_BYTES = 64 << 20
+# as the batch-one head. 33 MB from HBM, a row without the norm: 12.1 us on the
+# strips, 10.2 on the head (8.7 / 10.6 where the last pass left all of it cached,
+# which a whole model's other weights do not).
+STREAM_HEAD_BYTES = 16 << 20
 ARGMAX_ROWS = 32  # rows per 8-bit head launch (HTN_GEMM_TILES_ARGMAX_ROWS)
 TILE_ROWS = 256
 # A plain store (QKV) of LIBRARY_ROWS rows goes to the library, a residual

@@ -145,16 +145,16 @@ def test_residual_norm_rows_off_the_tiles(rows, n, k, layout):
         out.float(), (n,), gain.float(), 1e-6), atol=2e-2, rtol=2e-2)
 
 
-def test_small_vocabularies_keep_cached_loads():
+def test_small_vocabularies_stay_on_the_strips():
     def vocabulary(v, k):
         return torch.empty(v, k, dtype=torch.bfloat16, device="meta")
-    assert not RW.streams_head(vocabulary(32767, 1024)) and RW.streams_head(vocabulary(32768, 1024))
+    assert not RW.streams_head(vocabulary(8191, 1024)) and RW.streams_head(vocabulary(8192, 1024))
     codes, scale = torch.empty(16, 64, dtype=torch.uint8), torch.empty(16)
     assert RW.streams_head(RW.QuantizedWeight(codes, scale, "int8"))
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("vocab", [32767, 32768])  # either side of the streamed size
+@pytest.mark.parametrize("vocab", [8191, 8192])  # either side of the streamed size
 @pytest.mark.parametrize("rows", [1, 3, 15, 16, 17, 40])
 def test_greedy_rows_around_the_streamed_size(vocab, rows):
     x, w = matrix(rows, 1024, "plain", "cuda"), matrix(vocab, 1024, "plain", "cuda", 1)
