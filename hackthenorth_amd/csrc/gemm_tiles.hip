@@ -90,14 +90,19 @@ struct TileArgs {
 // rotated and past the caches (one row tile) 6.7.
 constexpr int kRotate = 37;
 // Weights of this size or more are streamed past the caches by the tiles of at
-// most 48 rows, and from kStreamOnceBytes on where a single row tile reads them.
+// most 48 rows, bf16 ones of any size from kStreamRows rows on.
 // From HBM streaming is faster: 4B int8, one tile, QKV of 15.7 MB 10.1 -> 9.3
 // us, O of 10.5 MB 11.4 -> 10.6; 8B at 32 rows in two tiles, O 15.0 -> 14.5,
-// down 35.7 -> 34.5. A small model's weights are still in the last-level cache
-// from the pass before (100 MB of them read in turn, 0.6B at 48 rows: QKV 6.4
-// cached / 8.2 streamed, gate/up of 12.6 MB 6.5 / 8.2; from HBM 8.3 / 8.0 and
-// 8.4 / 8.1).
-constexpr long kStreamBytes = 16L << 20, kStreamOnceBytes = 10L << 20;
+// down 35.7 -> 34.5. Smaller weights belong to small models, where the last-level
+// cache still holds a part from the pass before: the more, the less the larger
+// ones put there. Three 0.6B models' 125 MB in turn, rows: all cached / from
+// 10 MB on (gate/up) / all streamed: 40 rows 152 / 146 / 153 us, 64 157 / 152 /
+// 159, 128 170 / 161 / 174, 200 187 / 178 / 189; one model alone 140 / 147 / 155
+// and 171 / 177 / 189. From 256 rows on gate/up goes through the library, whose
+// loads fill the cache, and the rest is streamed: 256 rows 218 / 214 / 208, 300
+// 240 / 239 / 231, 400 255 / 255 / 252 (alone 193 / 192 / 207 and 234 for each).
+// 8-bit gate/up stays here: 256 rows 206 / 205 / 211, 300 229 / 228 / 233.
+constexpr long kStreamBytes = 10L << 20, kStreamRows = 256;
 constexpr int kMinSplitSteps = 8;     // k steps each split keeps at least
 constexpr int kMaxSplit = 12;
 
@@ -671,9 +676,9 @@ long tiles_scratch_bytes(const TilePlan& p, long rows) {
 
 // Whether tiles of one wave along the rows load a [n, k] weight (twice n rows
 // for SwiGLU) past the caches.
-bool streamed(long mtiles, long n, long k, int epilogue, int format) {
+bool streamed(long rows, long n, long k, int epilogue, int format) {
   const long bytes = (epilogue == HTN_EPI_SWIGLU ? 2 : 1) * n * k * (format == 0 ? 2 : 1);
-  return bytes >= (mtiles == 1 ? kStreamOnceBytes : kStreamBytes);
+  return bytes >= kStreamBytes || (format == 0 && rows >= kStreamRows);
 }
 
 template <int EPI, int WM, int WN, int NT, int WF, int AUX>
@@ -694,7 +699,7 @@ int launch_shape(TileArgs& a, long blocks, hipStream_t st) {
   constexpr int TM = Shape<WM, WN, NT, WF>::kTm;
   a.mtiles = (a.M + TM - 1) / TM;
   if constexpr (WM == 1) {
-    if (streamed(a.mtiles, a.N, a.K, EPI, WF))
+    if (streamed(a.M, a.N, a.K, EPI, WF))
       return launch_policy<EPI, WM, WN, NT, WF, 2>(a, blocks, st);
   }
   return launch_policy<EPI, WM, WN, NT, WF, 0>(a, blocks, st);
@@ -848,7 +853,7 @@ extern "C" int htn_gemm_tiles_plan(int64_t rows, int64_t n, int64_t k, int epilo
   plan[0] = static_cast<int32_t>(tm);
   plan[1] = 32 * p.wm * p.wn;
   plan[2] = p.ksplit;
-  plan[3] = p.wm == 1 && streamed((rows + tm - 1) / tm, n, k, epilogue, weight_format);
+  plan[3] = p.wm == 1 && streamed(rows, n, k, epilogue, weight_format);
   return HTN_OK;
 }
 

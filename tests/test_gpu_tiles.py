@@ -32,7 +32,7 @@ COVER = [(523, 528, 64), (1353, 16, 1792), (2, 13688, 768), (2, 1992, 5312), (18
          (34, 6848, 2112), (1227, 1032, 3840), (198, 14112, 6976), (1337, 5632, 64),
          (42, 22944, 704), (293, 1416, 8256), (1839, 1096, 9472), (17, 17000, 640),
          (653, 13320, 64), (696, 16504, 64), (67, 568, 3584), (397, 320, 6784), (884, 552, 7360),
-         (1375, 4240, 64), (196, 2944, 3328), (17, 12296, 448), (235, 5448, 6784)]
+         (1375, 4240, 64), (196, 2944, 3328), (17, 12296, 448), (235, 5448, 6784), (33, 11600, 64)]
 
 
 def bf16(seed, *shape, std=1.0):
